@@ -1,0 +1,125 @@
+"""BiCGStab iterated inside one launch (csrc/group.hip): sizes at the edges of
+its work-groups (512 faces; 256 for three species or hexahedra), remainders,
+the smallest systems, both precisions, both face orders, batches, and the
+launched iteration that takes over when a wait in the kernel gives up.  Solved
+to 1e-13, so the oracle's solution is met to 1e-10 (the parity bar)."""
+import ctypes as C
+
+import numpy as np
+import pytest
+
+from mhfem_amd import capi, problems
+import pyoracle
+
+pytestmark = pytest.mark.gpu
+
+
+def rel(a, b):
+    return np.linalg.norm(a - b) / max(np.linalg.norm(b), 1e-300)
+
+
+CASES = {
+    # 5, 456, 533, 1008 and 2080 faces
+    "tri1": lambda: problems.heat_2d(s=1, dt=1e-3),
+    "tri12": lambda: problems.heat_2d(s=12, dt=1e-3),
+    "tri13": lambda: problems.heat_2d(s=13, dt=1e-3),
+    "tri18_n2": lambda: problems.adr_2d(s=18, n=2),
+    "tri26_n3": lambda: problems.adr_2d(s=26, n=3),
+    # 480, 1012 and 41 faces
+    "quad15": lambda: problems.heat_quads(s=15),
+    "quad22_n2": lambda: problems.adr_quads(s=22, n=2),
+    "edge40": lambda: problems.adr_1d(s=40, n=2),
+    # 18, 378, 864, 1650 and 6528 faces
+    "tet1": lambda: problems.darcy_3d(s=1, preconditioner="diagonal"),
+    "tet3": lambda: problems.darcy_3d(s=3, preconditioner="diagonal"),
+    "tet4_n2": lambda: problems.adr_3d(s=4, n=2, preconditioner="diagonal"),
+    "tet5_n3": lambda: problems.adr_3d(s=5, n=3, preconditioner="diagonal"),
+    "tet8": lambda: problems.darcy_3d(s=8, preconditioner="diagonal", shuffle_cells=3),
+    # 756, 756 and 450 faces
+    "hex6": lambda: problems.adr_hexes(s=6, n=1),
+    "hex6_n2": lambda: problems.adr_hexes(s=6, n=2),
+    "hex5_n3": lambda: problems.adr_hexes(s=5, n=3),
+}
+
+
+def _steps(pr, s, o, steps=2):
+    t = 0.0
+    for k in range(steps):
+        st = s.step(t, pr.dt)
+        o.step(t, pr.dt, tol=1e-13)
+        t += pr.dt
+        assert st.converged and st.iterations > 0
+        assert rel(s.get_array("Z_iF"), o.array("Z_iF")) < 1e-10, k
+        assert rel(s.get_array("Z_iK"), o.array("Z_iK")) < 1e-10, k
+
+
+@pytest.mark.parametrize("groups", [0, 1])
+@pytest.mark.parametrize("precision", ["fp64", "fp32-reliable", "fp32-refined"])
+@pytest.mark.parametrize("case", sorted(CASES))
+def test_one_launch_matches_oracle(case, precision, groups):
+    print(f"\n[group] {case} {precision} groups {groups}", flush=True)
+    pr = CASES[case]()
+    s = capi.Solver(pr, preconditioner="diagonal", tol=1e-13, precision=precision, inner_tol=0.03, face_groups=groups)
+    _steps(pr, s, pyoracle.Oracle(pr))
+    s.close()
+
+
+@pytest.mark.parametrize("precision", ["fp64", "fp32-reliable"])
+def test_a_wait_that_gives_up_hands_over(precision):
+    """With a bound of zero the first wait between two work-groups gives up:
+    the solve is finished by the launched iteration, and so are the next ones."""
+    pr = problems.adr_3d(s=6, n=2, preconditioner="diagonal")
+    print(f"\n[group] handed over, {precision}", flush=True)
+    s = capi.Solver(pr, preconditioner="diagonal", tol=1e-13, precision=precision, inner_tol=0.03)
+    fn = capi.lib().mhfem_internal_group_wait
+    fn.argtypes = [C.c_void_p, C.c_ulonglong]
+    assert fn(s.ctx, 0) == 0
+    _steps(pr, s, pyoracle.Oracle(pr), steps=3)
+    s.close()
+
+
+def test_batch_larger_than_the_chip():
+    """More work-groups than fit at once: segments start in turn."""
+    members = [problems.ensemble_member(sd, 40 + k) for k, sd in enumerate([150, 20, 90, 150, 150, 7, 150])]
+    batch = problems.concatenate(members)
+    s = capi.Solver(batch, tol=1e-12)
+    co, fo = s.batch_info()
+    assert fo[-1] > 2 * 131072
+    s.step(0.0, batch.dt)
+    rp, col, val, rhs = s.export_system()
+    x = s.get_array("Z_iF")
+    r = rhs - np.add.reduceat(val * x[col], rp[:-1])
+    for k in range(len(members)):
+        a, b = fo[k], fo[k + 1]
+        assert np.linalg.norm(r[a:b]) < 2e-12 * np.linalg.norm(rhs[a:b]), k
+    s.close()
+
+
+def test_overlapping_contexts():
+    """Two contexts solve at the same time on their own streams."""
+    import threading
+
+    prs = [problems.heat_2d(s=60, dt=1e-3), problems.darcy_3d(s=9, preconditioner="diagonal")]
+    oracles = [pyoracle.Oracle(p) for p in prs]
+    for p, o in zip(prs, oracles):
+        o.step(0.0, p.dt, tol=1e-13)
+    solvers = [capi.Solver(p, preconditioner="diagonal", tol=1e-13) for p in prs]
+    errors = []
+
+    def work(p, s, o):
+        for _ in range(5):
+            s.set_array("Z_iK", p.Z_iK0)
+            capi.lib().mhfem_init(s.ctx)
+            s.step(0.0, p.dt)
+            e = rel(s.get_array("Z_iF"), o.array("Z_iF"))
+            if not e < 1e-10:
+                errors.append(e)
+
+    threads = [threading.Thread(target=work, args=a) for a in zip(prs, solvers, oracles)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not errors
+    for s in solvers:
+        s.close()

@@ -1190,6 +1190,17 @@ int mhfem_guess_gradient(mhfem_ctx *ctx, const uint16_t *features, const float *
     });
 }
 
+// Test aid, not part of the interface: the bound of the waits of the
+// one-launch BiCGStab in 100 MHz ticks (0: every wait gives up at once and
+// the solve is finished by the launched iteration).
+extern "C" int mhfem_internal_group_wait(mhfem_ctx *ctx, unsigned long long ticks)
+{
+    return guarded(ctx, [&](Ctx &c) {
+        if (!c.system_ready) throw Error{MHFEM_E_STATE, "linear system not set up"};
+        krylov_set_group_wait(*c.krylov, ticks);
+    });
+}
+
 int mhfem_batch_stats(mhfem_ctx *ctx, int32_t *iterations, double *residues, int count)
 {
     return guarded(ctx, [&](Ctx &c) {

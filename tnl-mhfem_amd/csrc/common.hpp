@@ -27,7 +27,7 @@ void set_global_error(const std::string &msg);
 // device scalar slots of the Krylov solver (per segment)
 enum Slot {
     S_RHO = 0, S_RHO_OLD, S_ALPHA, S_OMEGA, S_BETA, S_RAST_SQ, S_BNORM, S_RESID, S_TOL, S_IT,
-    S_DONE, S_RESTART, S_MAXIT, S_D0, S_D1, S_D2, S_D3, S_TOLABS, S_DELTA, S_BFIX, S_BREAK, NSLOTS = 32
+    S_DONE, S_RESTART, S_MAXIT, S_D0, S_D1, S_D2, S_D3, S_TOLABS, S_DELTA, S_BFIX, S_BREAK, S_FAIL, NSLOTS = 32
 };
 // a segment's solve has stopped (converged, failed or waiting for a restart):
 // kernels queued behind it return at once
@@ -361,6 +361,30 @@ void launch_geometry(Ctx &c);
 void launch_fill_b(Ctx &c);
 void launch_fill_R(Ctx &c);
 void launch_zero_double(Ctx &c, double *p, size_t n);
+
+// group.hip
+// One work-group's share of a segment: the positions [p0, p1) of the groups'
+// face order, rank in the group
+struct GroupTask {
+    int seg, rank, p0, p1;
+};
+struct GroupPlan {
+    int total = 0;  // work-groups, 0: the system does not fit on the chip
+    int threads = 0, width = 0, nslots = 0;
+    DBuf<GroupTask> task;
+    DBuf<int> seg;       // int2 per segment
+    DBuf<int> face, pos; // the groups' face order and its inverse
+    DBuf<double> slots;
+    DBuf<int> counters;  // ticket, beat
+    DBuf<char> pub;
+    int cooldown = 0;    // solves left that iterate by launches after a wait gave up
+    unsigned long long wait_ticks = 500000;  // 5 ms of the 100 MHz counter without any iteration in the launch
+};
+bool group_plan(Ctx &c, GroupPlan &gp, bool fp32, int width);
+template <typename T>
+void group_iterate(Ctx &c, GroupPlan &gp, const SellView<T> &A, double *sc, T *x, T *r, T *p, const T *r_ast);
+void group_clear_failed(Ctx &c, double *sc, int nseg);
+void krylov_set_group_wait(Krylov &k, unsigned long long ticks);
 
 // krylov.hip
 Krylov *krylov_create(Ctx &c);

@@ -1,0 +1,711 @@
+// group.hip -- BiCGStab of systems that fit on the chip, one launch per
+// solve: every segment is iterated by a group of work-groups that stay
+// resident until it stops.
+//
+// What bounds the launched iteration (krylov.hip) on such systems is not
+// memory: six to eight dependent launches of a few microseconds each, and a
+// host read of the flags per batch, 37-48 us per iteration whatever the size
+// below about 200,000 unknowns.  Here a lane owns a face.  Its matrix rows,
+// its p and r, and copies of its neighbours' p and r live in registers (x and
+// r* in LDS); an iteration is the merged recurrence (FIN_*_MERGED) with two
+// exchanges.  In each the lanes publish one vector (Ap, then As), the
+// work-groups publish their partial dot products, and every work-group reads
+// all partial sums and the published values of its neighbours; each lane then
+// updates the copies of its neighbours' vectors with the arithmetic of their
+// owners, so p and s are never exchanged themselves.
+//
+// * Published values are their own flags (device.hpp): no fence, no counter,
+//   and the gather of the neighbours overlaps the reduction.  There are
+//   GROUP_ROT copies; one is cleared by its owner once every work-group has
+//   posted the epoch after it, three epochs before it is used again.
+// * All work-groups add the partial sums in one order, so all take the same
+//   decisions and leave the loop together.
+// * Faces are taken along a space-filling curve (group_order): most
+//   neighbours are in the same work-group and come through LDS.
+// * Work-groups take their share by ticket, the segments' shares in a row,
+//   largest segment first: the earliest unfinished segment always has all its
+//   work-groups resident once earlier ones have left, so a batch may have
+//   many more work-groups than fit at once.
+// * Nothing else on the GPU is waited for: when another launch holds places
+//   that a segment needs and neither gets on, no iteration of this launch
+//   happens for 5 ms and the waits give up.  The segment is marked, every
+//   work-group leaves, and the host restarts it with the launched iteration
+//   from the iterate it has (and keeps to that for the next solves).
+//
+// Measured (MI355X, whole trajectories as in perf/cases.py, launched -> one
+// launch): 64 x 64 x 2 triangles, 3 steps 3.21 -> 0.59 ms; 201 x 201 x 2,
+// 2 steps 6.37 -> 1.50 ms; 21^3 x 6 tetrahedra n = 1, 2 steps 17.7 -> 2.71 ms
+// (48 -> 7.2 us per iteration); 20^3 x 6 n = 2, FP32, 6 steps 50.5 -> 13.1 ms;
+// 20^3 voxels n = 3, 6.77 -> 1.93 ms; 32 ragged 2-D instances 40.8 -> 20.4 ms.
+// An exchange takes 3.0-3.7 us with 200 work-groups (2 us with 25): 0.5 us of
+// arithmetic, 0.4 us of work-group sums, 2 us from the post of the slowest
+// work-group to its sum in every other one.  Tried: neighbours polled only
+// after the sums are in (10 us per iteration instead of 8); wavefronts that
+// sleep before they poll (no change); the partial sums in one copy instead of
+// GROUP_REP (5 % slower at 200 work-groups); faces in the mesh order (gathers
+// 2.3 us instead of 1.6).
+#include <algorithm>
+#include <type_traits>
+
+#include "common.hpp"
+#include "device.hpp"
+
+namespace mhfem {
+
+constexpr int GROUP_ROT = 4;  // rotating copies of the published vectors and partial sums
+constexpr int GROUP_REP = 8;  // copies of the partial sums, each read by every 8th work-group
+constexpr int GROUP_ND = 4;   // dot products of a reduction, at most
+
+// partial sums a wavefront adds, per dot product: BS / 256 wavefronts for each
+// of GROUP_ND dots cover the largest group (one work-group per CU of 256)
+constexpr int group_slots(int bs) { return bs <= 256 ? 256 : 128; }
+
+struct GroupView {
+    int total;               // work-groups of the launch
+    int64_t rows;
+    const GroupTask *task;   // per ticket
+    const int *face, *pos;   // the face at a position of the groups' order, and its inverse
+    const int2 *seg;         // per segment: first slot (of GROUP_ROT * GROUP_ND * groups), groups
+    int *ticket;             // [0]
+    unsigned *beat;          // [0]: iterations of every segment of the launch
+    double *slots;
+    double *sc;
+    unsigned long long wait_ticks;  // bound of a wait, 0: every wait gives up at its first pause
+};
+
+// Values of one face moved through memory as 8- or 4-byte words with
+// device-coherent accesses; a component that still holds the sentinel has not
+// been written yet.
+template <typename T, int N>
+struct FaceWords {
+    using U = std::conditional_t<(sizeof(T) * N) % 8 == 0, unsigned long long, unsigned int>;
+    static constexpr int M = (int)(sizeof(T) * N / sizeof(U));
+    union {
+        U w[M];
+        T v[N];
+    };
+    __device__ FaceWords() {}
+};
+template <typename T, int N>
+__device__ __forceinline__ void publish(T *dst, const Pack<T, N> &a)
+{
+    FaceWords<T, N> f;
+#pragma unroll
+    for (int i = 0; i < N; i++) f.v[i] = is_sentinel(a.v[i]) ? (T)__builtin_nan("") : a.v[i];
+    auto *q = reinterpret_cast<typename FaceWords<T, N>::U *>(dst);
+#pragma unroll
+    for (int m = 0; m < FaceWords<T, N>::M; m++) coherent_store(q + m, f.w[m]);
+}
+template <typename T, int N>
+__device__ __forceinline__ Pack<T, N> look(const T *src)
+{
+    FaceWords<T, N> f;
+    auto *q = reinterpret_cast<const typename FaceWords<T, N>::U *>(src);
+#pragma unroll
+    for (int m = 0; m < FaceWords<T, N>::M; m++) f.w[m] = coherent_load(q + m);
+    Pack<T, N> a;
+#pragma unroll
+    for (int i = 0; i < N; i++) a.v[i] = f.v[i];
+    return a;
+}
+template <typename T, int N>
+__device__ __forceinline__ void unpublish(T *dst)
+{
+    FaceWords<T, N> f;
+#pragma unroll
+    for (int i = 0; i < N; i++) f.v[i] = sentinel_value<T>();
+    auto *q = reinterpret_cast<typename FaceWords<T, N>::U *>(dst);
+#pragma unroll
+    for (int m = 0; m < FaceWords<T, N>::M; m++) coherent_store(q + m, f.w[m]);
+}
+
+// a value every lane of the wavefront holds, moved to scalar registers
+__device__ __forceinline__ double uniform(double v)
+{
+    const unsigned long long b = __builtin_bit_cast(unsigned long long, v);
+    const unsigned lo = __builtin_amdgcn_readfirstlane((unsigned)b), hi = __builtin_amdgcn_readfirstlane((unsigned)(b >> 32));
+    return __builtin_bit_cast(double, (unsigned long long)hi << 32 | lo);
+}
+
+// every memory access issued so far is complete (the builtin, so that the
+// compiler's own count of outstanding accesses starts at zero here)
+__device__ __forceinline__ void memory_done()
+{
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0)
+    asm volatile("" ::: "memory");
+}
+
+// bounded waiting: gives up once nothing in the launch has iterated for
+// GROUP_WAIT_TICKS, or a work-group of the segment has given up
+struct GroupWait {
+    const GroupView &g;
+    double *fail;  // the segment's S_FAIL
+    unsigned long long t0 = 0;
+    unsigned beat = 0;
+    int idle = 0;
+    bool gave_up = false;
+    __device__ GroupWait(const GroupView &v, double *f) : g(v), fail(f) {}
+    __device__ __forceinline__ bool pause()
+    {
+        __builtin_amdgcn_s_sleep(1);
+        if ((++idle & 63) == 0 || g.wait_ticks == 0) {
+            const unsigned long long now = __builtin_amdgcn_s_memrealtime();
+            const unsigned b = coherent_load(g.beat);
+            if (t0 == 0 || b != beat) {
+                t0 = now;
+                beat = b;
+            } else if (now - t0 > g.wait_ticks) {
+                gave_up = true;
+            }
+            if (g.wait_ticks == 0) gave_up = true;
+            if (coherent_load(fail) != 0.0) gave_up = true;
+            if (gave_up) coherent_store(fail, 1.0);
+        }
+        return gave_up;
+    }
+};
+
+template <typename T, int N, int W, int BS, bool HOLD>
+__global__ void __launch_bounds__(BS) k_bicg_group(SellView<T> A, GroupView g, T *__restrict__ xg, T *__restrict__ rg,
+                                                   T *__restrict__ pg, const T *__restrict__ r_ast, T *pub)
+{
+    constexpr int NW = BS / 64, SLOTS = group_slots(BS);
+    __shared__ int s_ticket, s_fail;
+    __shared__ double part[2][GROUP_ND][NW], tot[2][GROUP_ND][NW / GROUP_ND];
+    __shared__ Pack<T, N> mine[2][BS];  // the work-group's own published values
+    __shared__ Pack<T, N> own[2][BS];   // x and r* of each lane
+    const int tid = threadIdx.x, lane = tid & 63, wid = __builtin_amdgcn_readfirstlane(tid >> 6);
+    if (tid == 0) {
+        s_ticket = atomicAdd(g.ticket, 1);
+        s_fail = 0;
+    }
+    if (tid < 2 * GROUP_ND * (NW / GROUP_ND)) (&tot[0][0][0])[tid] = 0.0;  // chunks past the group stay zero
+    __syncthreads();
+    const int ticket = __builtin_amdgcn_readfirstlane(s_ticket);
+    if (ticket >= g.total) return;
+    const GroupTask task = g.task[ticket];
+    double *sc = g.sc + (int64_t)task.seg * NSLOTS;
+    if (halted(sc)) return;
+    const int G = g.seg[task.seg].y;
+    double *slots = g.slots + g.seg[task.seg].x;
+    const int at = task.p0 + tid;  // position in the groups' order
+    const bool valid = at < task.p1;
+    const int f = valid ? g.face[at] : 0;
+
+    // ---- the face's matrix rows and its state; neighbours' p and r
+    int col[W];  // the neighbour's row in the published vector, or -1 - its lane when this work-group has it
+    Pack<T, N * N> val[HOLD ? W : 1];
+    Pack<T, (N > 1 ? N * (N - 1) : 1)> dg;
+    Pack<T, N> p, r, pn[W], rn[W];
+    int w = 0;
+#pragma unroll
+    for (int i = 0; i < N; i++) p.v[i] = r.v[i] = T(0);
+    if constexpr (N > 1) {
+#pragma unroll
+        for (int i = 0; i < N * (N - 1); i++) dg.v[i] = T(0);
+    }
+    int64_t base = 0;
+    if (valid) {
+        base = A.slice_ptr[f >> 6] + (f & 63);
+        w = A.slice_width[f >> 6];
+    }
+    unsigned remote = 0;  // neighbours in other work-groups
+    bool alone = true;    // no neighbour but itself (padding)
+#pragma unroll
+    for (int k = 0; k < W; k++) {
+        col[k] = k < w ? A.col[base + (int64_t)k * 64] : f;
+        if constexpr (HOLD) {
+#pragma unroll
+            for (int i = 0; i < N * N; i++) val[k].v[i] = T(0);
+        }
+#pragma unroll
+        for (int i = 0; i < N; i++) pn[k].v[i] = rn[k].v[i] = T(0);
+        if (k < w) {
+            if constexpr (HOLD) val[k] = ld<T, N * N>(A.val + (base + (int64_t)k * 64) * (N * N));
+            pn[k] = ld<T, N>(pg + (int64_t)col[k] * N);
+            rn[k] = ld<T, N>(rg + (int64_t)col[k] * N);
+        }
+        alone = alone && col[k] == f;
+        col[k] = k < w ? g.pos[col[k]] : task.p0;
+        if (col[k] < task.p0 || col[k] >= task.p1) remote |= 1u << k;
+        else col[k] = -1 - (col[k] - task.p0);
+    }
+    // The pattern is symmetric but for faces without neighbours (all rows
+    // Dirichlet), which their neighbours read: those faces and the ones that
+    // read other work-groups' faces are published.
+    const bool shared_face = valid && (remote != 0 || alone);
+    own[0][tid] = own[1][tid] = p;
+    if (valid) {
+        p = ld<T, N>(pg + (int64_t)f * N);
+        r = ld<T, N>(rg + (int64_t)f * N);
+        own[0][tid] = ld<T, N>(xg + (int64_t)f * N);
+        own[1][tid] = ld<T, N>(r_ast + (int64_t)f * N);
+        if constexpr (N > 1) dg = ld<T, N *(N - 1)>(A.val + A.diag_base + (int64_t)f * N * (N - 1));
+    }
+    double rho = uniform(sc[S_RHO]), rho_old = uniform(sc[S_RHO_OLD]), alpha = uniform(sc[S_ALPHA]),
+           omega = uniform(sc[S_OMEGA]), beta = uniform(sc[S_BETA]);
+    double resid = 0.0, it = uniform(sc[S_IT]), brk = uniform(sc[S_BREAK]);
+    double inv_pap = 0.0;  // alpha / rho
+    const double bnorm = uniform(sc[S_BNORM]), tol = uniform(sc[S_TOL]), maxit = uniform(sc[S_MAXIT]),
+                 rast_sq = uniform(sc[S_RAST_SQ]);
+    double done = 0.0, restart = 0.0;
+    const double eps2 = 2.220446049250313e-16 * 2.220446049250313e-16;
+    // every read of the arrays that the segment's work-groups write at the
+    // end is complete before this work-group's first partial sums go out
+    memory_done();
+
+    auto product = [&](const Pack<T, N> &own, const Pack<T, N>(&nb)[W]) {
+        Pack<T, N> y = own;
+        if constexpr (N > 1) {
+#pragma unroll
+            for (int i = 0; i < N; i++)
+#pragma unroll
+                for (int j = 0; j < N; j++)
+                    if (j != i) y.v[i] += dg.v[i * (N - 1) + (j < i ? j : j - 1)] * own.v[j];
+        }
+#pragma unroll
+        for (int k = 0; k < W; k++) {
+            if constexpr (!HOLD) {
+                if (k < w) val[0] = ld<T, N * N>(A.val + (base + (int64_t)k * 64) * (N * N));
+            }
+            if (HOLD || k < w) {
+#pragma unroll
+                for (int i = 0; i < N; i++)
+#pragma unroll
+                    for (int j = 0; j < N; j++) y.v[i] += val[HOLD ? k : 0].v[i * N + j] * nb[k].v[j];
+            }
+        }
+        return y;
+    };
+    GroupWait wait(g, sc + S_FAIL);
+    int e = 0;  // epoch: one per reduction
+    // publishes y, sums the partials of ND dots over the group into tot and
+    // gathers the neighbours' published values; false: a wait gave up
+    auto exchange = [&](const Pack<T, N> &y, auto &acc, auto NDC, Pack<T, N>(&nb)[W]) {
+        constexpr int ND = decltype(NDC)::value;
+        const int rot = e & (GROUP_ROT - 1), par = e & 1;
+        T *pb = pub + (int64_t)rot * g.rows;
+        if (shared_face) publish<T, N>(pb + (int64_t)at * N, y);
+        mine[par][tid] = y;
+        const double ws = sums_wave<ND>(acc);
+        if ((lane & (64 / ND - 1)) == 0) part[par][lane / (64 / ND)][wid] = ws;
+        __syncthreads();
+        if (tid < ND * GROUP_REP) {
+            double s = part[par][tid % ND][0];
+#pragma unroll
+            for (int q = 1; q < NW; q++) s += part[par][tid % ND][q];
+            if (is_sentinel(s)) s = __builtin_nan("");
+            coherent_store(slots + (((int64_t)(tid / ND) * GROUP_ROT + rot) * GROUP_ND + tid % ND) * G + task.rank, s);
+        }
+#pragma unroll
+        for (int k = 0; k < W; k++)
+            if (col[k] < 0) nb[k] = mine[par][-1 - col[k]];
+        // Polls for the neighbours' values in other work-groups and, in wave
+        // d + ND c, for the sums of dot d of SLOTS work-groups: each round looks
+        // at everything still missing with one wait.
+        unsigned pend = remote, pd = 0;
+        const int dot = wid & (ND - 1), chunk = wid / ND * SLOTS;
+        const double *row =
+            slots + (((int64_t)(task.rank % GROUP_REP) * GROUP_ROT + rot) * GROUP_ND + dot) * G + chunk;
+        double v[SLOTS / 64];
+#pragma unroll
+        for (int q = 0; q < SLOTS / 64; q++) {
+            v[q] = 0.0;
+            if (chunk + q * 64 + lane < G) pd |= 1u << q;
+        }
+        for (;;) {
+#pragma unroll
+            for (int k = 0; k < W; k++)
+                if (pend >> k & 1u) nb[k] = look<T, N>(pb + (int64_t)col[k] * N);
+#pragma unroll
+            for (int q = 0; q < SLOTS / 64; q++)
+                if (pd >> q & 1u) v[q] = coherent_load(row + q * 64 + lane);
+#pragma unroll
+            for (int k = 0; k < W; k++) {
+                bool there = true;
+#pragma unroll
+                for (int i = 0; i < N; i++) there = there && !is_sentinel(nb[k].v[i]);
+                if (there) pend &= ~(1u << k);
+            }
+#pragma unroll
+            for (int q = 0; q < SLOTS / 64; q++)
+                if (!is_sentinel(v[q])) pd &= ~(1u << q);
+            if (!__any((pend | pd) != 0)) break;
+            if (wait.pause()) {
+                if (lane == 0) s_fail = 1;
+                break;
+            }
+        }
+        wait.t0 = 0;
+        if (chunk < G) {
+            double one[1] = {v[0]};
+#pragma unroll
+            for (int q = 1; q < SLOTS / 64; q++) one[0] += v[q];
+            const double s = sums_wave<1>(one);
+            if (lane == 0) tot[par][dot][wid / ND] = s;
+        }
+        // the clearing stores of the previous epoch are complete before the
+        // work-group posts its next partial sums
+        memory_done();
+        __syncthreads();
+        // every work-group has posted this epoch, so none still reads the
+        // previous one: its copies are cleared, for epoch e + 3
+        const int old = (e + GROUP_ROT - 1) & (GROUP_ROT - 1);
+        if (shared_face) unpublish<T, N>(pub + (int64_t)old * g.rows + (int64_t)at * N);
+        if (tid < GROUP_ND * GROUP_REP)
+            coherent_store(slots + (((int64_t)(tid / GROUP_ND) * GROUP_ROT + old) * GROUP_ND + tid % GROUP_ND) * G +
+                               task.rank,
+                           sentinel_value<double>());
+        e++;
+        return s_fail == 0;
+    };
+    // a sum over the group, from its chunks
+    auto total = [&](int d) {
+        const int q = (e - 1) & 1;
+        double s = tot[q][d][0];
+#pragma unroll
+        for (int c = 1; c < NW / GROUP_ND; c++) s += tot[q][d][c];
+        return uniform(s);
+    };
+
+    bool ok = true;
+    for (;;) {
+        Pack<T, N> an[W], a2[W];
+        // ---- Ap, (Ap, r*), (r, r)
+        const Pack<T, N> Ap = product(p, pn);
+        const Pack<T, N> ra = own[1][tid];
+        double d2[2] = {0.0, 0.0};
+#pragma unroll
+        for (int i = 0; i < N; i++) {
+            d2[0] += (double)Ap.v[i] * (double)ra.v[i];
+            d2[1] += (double)r.v[i] * (double)r.v[i];
+        }
+        if (!valid) d2[0] = d2[1] = 0.0;
+        ok = exchange(Ap, d2, std::integral_constant<int, 2>{}, an);
+        if (!ok) break;
+        {
+            const double D0 = total(0), D1 = total(1);
+            resid = uniform(sqrt(D1) / bnorm);
+            if (!(resid >= tol) || it >= maxit) {
+                done = 1.0;
+                break;
+            }
+            if (brk != 0.0) {
+                brk = 0.0;
+                restart = 1.0;
+                break;
+            }
+            const double a = uniform(rho / D0);
+            if (!(fabs(D0) > 0.0) || !isfinite(a)) {
+                restart = 1.0;
+                it += 1.0;
+                if (it >= maxit) done = 1.0;
+                break;
+            }
+            alpha = a;
+            inv_pap = uniform(1.0 / D0);
+        }
+        const T al = (T)alpha;
+        Pack<T, N> s;
+#pragma unroll
+        for (int i = 0; i < N; i++) s.v[i] = r.v[i] - al * Ap.v[i];
+#pragma unroll
+        for (int k = 0; k < W; k++)
+#pragma unroll
+            for (int i = 0; i < N; i++) rn[k].v[i] = rn[k].v[i] - al * an[k].v[i];
+        // ---- As, (As, s), (As, As), (As, r*), (s, r*)
+        const Pack<T, N> As = product(s, rn);
+        const Pack<T, N> rb = own[1][tid];
+        double d4[4] = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+        for (int i = 0; i < N; i++) {
+            const double av = As.v[i], sv = s.v[i], rv = rb.v[i];
+            d4[0] += av * sv;
+            d4[1] += av * av;
+            d4[2] += av * rv;
+            d4[3] += sv * rv;
+        }
+        if (!valid) d4[0] = d4[1] = d4[2] = d4[3] = 0.0;
+        ok = exchange(As, d4, std::integral_constant<int, 4>{}, a2);
+        if (!ok) break;
+        {
+            const double D[4] = {total(0), total(1), total(2), total(3)};
+            // beta = (rho / rho_old) (alpha / omega) with alpha / rho_old = 1 / (r*, Ap)
+            const double om = uniform(D[1] > 0 ? D[0] / D[1] : 0.0), inv_om = uniform(D[1] / D[0]);
+            const double rn_ = uniform(D[3] - om * D[2]);
+            omega = om;
+            it += 1.0;
+            rho_old = rho;
+            rho = rn_;
+            if (!(fabs(rho) >= eps2 * rast_sq) || om == 0.0) {
+                beta = 0.0;
+                brk = 1.0;
+            } else {
+                beta = uniform((rho * inv_pap) * inv_om);
+            }
+        }
+        const T om = (T)omega, be = (T)beta;
+        Pack<T, N> x = own[0][tid];
+#pragma unroll
+        for (int i = 0; i < N; i++) {
+            x.v[i] += al * p.v[i] + om * s.v[i];
+            r.v[i] = s.v[i] - om * As.v[i];
+            p.v[i] = r.v[i] + be * (p.v[i] - om * Ap.v[i]);
+        }
+        own[0][tid] = x;
+#pragma unroll
+        for (int k = 0; k < W; k++)
+#pragma unroll
+            for (int i = 0; i < N; i++) {
+                rn[k].v[i] = rn[k].v[i] - om * a2[k].v[i];
+                pn[k].v[i] = rn[k].v[i] + be * (pn[k].v[i] - om * an[k].v[i]);
+            }
+        if (task.rank == 0 && tid == 0) atomicAdd(g.beat, 1u);
+    }
+    if (!ok) return;
+    if (valid) {
+        st<T, N>(xg + (int64_t)f * N, own[0][tid]);
+        st<T, N>(rg + (int64_t)f * N, r);
+        st<T, N>(pg + (int64_t)f * N, p);
+    }
+    if (task.rank == 0 && tid == 0) {
+        sc[S_RHO] = rho;
+        sc[S_RHO_OLD] = rho_old;
+        sc[S_ALPHA] = alpha;
+        sc[S_OMEGA] = omega;
+        sc[S_BETA] = beta;
+        sc[S_RESID] = resid;
+        sc[S_IT] = it;
+        sc[S_BREAK] = brk;
+        sc[S_DONE] = done;
+        sc[S_RESTART] = restart;
+    }
+}
+
+// sentinels in the published vectors and the slots, counters at zero
+template <typename T>
+__global__ void __launch_bounds__(256) k_group_prepare(int64_t pubn, T *pub, int slotn, double *slots, int *ticket,
+                                                       unsigned *beat)
+{
+    const int64_t stride = (int64_t)gridDim.x * 256, t = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    for (int64_t i = t; i < pubn; i += stride) pub[i] = sentinel_value<T>();
+    for (int64_t i = t; i < slotn; i += stride) slots[i] = sentinel_value<double>();
+    if (t == 0) {
+        *ticket = 0;
+        *beat = 0;
+    }
+}
+
+// segments whose waits gave up: the host restarts them from their iterate
+__global__ void k_group_failed(double *sc, int nseg)
+{
+    const int s = blockIdx.x * blockDim.x + threadIdx.x;
+    if (s >= nseg) return;
+    double *q = sc + (int64_t)s * NSLOTS;
+    if (q[S_FAIL] != 0.0) {
+        q[S_FAIL] = 0.0;
+        q[S_DONE] = 0.0;
+        q[S_RESTART] = 1.0;
+    }
+}
+
+namespace {
+
+template <typename F>
+void with_shape(int n, int width, F &&f)
+{
+    auto go = [&](auto NC) {
+        if (width <= 4) f(NC, std::integral_constant<int, 4>{});
+        else if (width <= 6) f(NC, std::integral_constant<int, 6>{});
+        else f(NC, std::integral_constant<int, 10>{});
+    };
+    if (n == 1) go(std::integral_constant<int, 1>{});
+    else if (n == 2) go(std::integral_constant<int, 2>{});
+    else go(std::integral_constant<int, 3>{});
+}
+// Registers of a lane, about: a work-group of 1024 threads has 128, of 512
+// 256, of 256 512 (part of them accumulation registers).  Shapes past 400
+// read the matrix from memory in each product instead.
+constexpr int lane_registers(int bytes, int n, int w) { return bytes / 4 * (n * (4 * w + 7) + n * n * (w + 1)) + w + 30; }
+constexpr int max_threads(int bytes, int n, int w)
+{
+    return lane_registers(bytes, n, w) <= 92 ? 1024 : lane_registers(bytes, n, w) <= 240 ? 512 : 256;
+}
+constexpr bool holds(int bytes, int n, int w) { return lane_registers(bytes, n, w) <= 400; }
+template <typename T, typename F>
+void with_threads(int bs, int n, int w, F &&f)
+{
+    with_shape(n, w, [&](auto NC, auto WC) {
+        constexpr int M = max_threads(sizeof(T), decltype(NC)::value, decltype(WC)::value);
+        if constexpr (M == 1024)
+            if (bs == 1024) return f(NC, WC, std::integral_constant<int, 1024>{});
+        f(NC, WC, std::integral_constant<int, (M < 512 ? M : 512)>{});
+    });
+}
+
+// The faces of every segment in Morton order of their positions (the lowest
+// corner of the first cell: a cell's faces stay together), so that a
+// work-group's faces are a compact piece of the mesh and few of their
+// neighbours belong to other work-groups.  Stable, by a radix sort of 33 bits.
+void group_order(const Ctx &c, std::vector<int> &face)
+{
+    for (int E = 0; E < c.F; E++) face[E] = E;
+    if (c.h_face_pos.size() != 3 * (size_t)c.F) return;
+    std::vector<uint64_t> key, other;
+    for (size_t s = 0; s + 1 < c.h_seg_faces.size(); s++) {
+        const int f0 = c.h_seg_faces[s], F = c.h_seg_faces[s + 1] - f0;
+        if (F < 2) continue;
+        const float *p = c.h_face_pos.data() + 3 * (size_t)f0;
+        float lo[3], hi[3], scale[3];
+        for (int d = 0; d < 3; d++) lo[d] = hi[d] = p[d];
+        for (int E = 0; E < F; E++)
+            for (int d = 0; d < 3; d++) {
+                lo[d] = std::min(lo[d], p[3 * (size_t)E + d]);
+                hi[d] = std::max(hi[d], p[3 * (size_t)E + d]);
+            }
+        for (int d = 0; d < 3; d++) scale[d] = hi[d] > lo[d] ? 2047.0f / (hi[d] - lo[d]) : 0.0f;
+        // bits 32.., the key; below, the face
+        auto spread = [](uint64_t v) {  // 11 bits to every third bit
+            v = (v | v << 16) & 0x30000ffull;
+            v = (v | v << 8) & 0x300f00full;
+            v = (v | v << 4) & 0x30c30c3ull;
+            return (v | v << 2) & 0x9249249ull;
+        };
+        key.resize(F);
+        other.resize(F);
+        for (int E = 0; E < F; E++) {
+            uint64_t m = 0;
+            for (int d = 0; d < 3; d++) {
+                const uint64_t q = (uint64_t)std::min(2047.0f, std::max(0.0f, (p[3 * (size_t)E + d] - lo[d]) * scale[d]));
+                m |= (spread(q & 1023) | (q >> 10) << 30) << d;
+            }
+            key[E] = m << 31 | (uint64_t)E;
+        }
+        for (int pass = 0; pass < 3; pass++) {
+            std::vector<int> count(2049, 0);
+            const int shift = 31 + 11 * pass;
+            for (int E = 0; E < F; E++) count[((key[E] >> shift) & 2047) + 1]++;
+            for (int b = 0; b < 2048; b++) count[b + 1] += count[b];
+            for (int E = 0; E < F; E++) other[count[(key[E] >> shift) & 2047]++] = key[E];
+            key.swap(other);
+        }
+        for (int E = 0; E < F; E++) face[f0 + E] = f0 + (int)(key[E] & 0x7fffffffull);
+    }
+}
+
+}  // namespace
+
+bool group_plan(Ctx &c, GroupPlan &gp, bool fp32, int width)
+{
+    gp.total = 0;
+    if (width > 10 || width < 1) return false;
+    const int cap_bs = [&] {
+        int m = 256;
+        with_shape(c.n, width, [&](auto NC, auto WC) {
+            m = max_threads(fp32 ? 4 : 8, decltype(NC)::value, decltype(WC)::value);
+        });
+        return m;
+    }();
+    int cus = 0;
+    MHFEM_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, c.device));
+    // 512 threads while one such work-group per CU holds every face (64 x 64
+    // x 2 triangles: 0.63 ms with 512, 0.76 ms with 1024); more faces take the
+    // largest the registers allow (32 ragged instances, 1.5 M faces: 26 ms
+    // with 512, 18 ms with 1024: fewer partial sums per face)
+    const int bs = c.F <= 512 * cus ? std::min(512, cap_bs) : cap_bs;
+    int per_cu = 0;
+    if (fp32)
+        with_threads<float>(bs, c.n, width, [&](auto NC, auto WC, auto BC) {
+            MHFEM_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(
+                &per_cu, (k_bicg_group<float, decltype(NC)::value, decltype(WC)::value, decltype(BC)::value, holds(4, decltype(NC)::value, decltype(WC)::value)>),
+                decltype(BC)::value, 0));
+        });
+    else
+        with_threads<double>(bs, c.n, width, [&](auto NC, auto WC, auto BC) {
+            MHFEM_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(
+                &per_cu, (k_bicg_group<double, decltype(NC)::value, decltype(WC)::value, decltype(BC)::value, holds(8, decltype(NC)::value, decltype(WC)::value)>),
+                decltype(BC)::value, 0));
+        });
+    // (and as many as the wavefronts of a work-group sum)
+    const long cap = std::min((long)per_cu * cus, (long)group_slots(bs) * (bs / 256));
+    std::vector<GroupTask> tasks;
+    const int nseg = (int)c.h_seg_faces.size() - 1;
+    std::vector<int2> segs(nseg);
+    std::vector<int> order(nseg);
+    for (int s = 0; s < nseg; s++) order[s] = s;
+    std::stable_sort(order.begin(), order.end(), [&](int a, int b) {
+        return c.h_seg_faces[a + 1] - c.h_seg_faces[a] > c.h_seg_faces[b + 1] - c.h_seg_faces[b];
+    });
+    auto split = [&](int F, int &G, int &fpw) {
+        G = std::max(1, (F + bs - 1) / bs);
+        fpw = std::min(bs, ((F + G - 1) / G + 63) / 64 * 64);
+        G = std::max(1, (F + fpw - 1) / std::max(1, fpw));
+    };
+    for (int s = 0; s < nseg; s++) {
+        int G, fpw;
+        split(c.h_seg_faces[s + 1] - c.h_seg_faces[s], G, fpw);
+        if (G > cap) return false;
+    }
+    // positions: each segment's faces along a space-filling curve
+    std::vector<int> face(c.F), pos(c.F);
+    group_order(c, face);
+    for (int q = 0; q < c.F; q++) pos[face[q]] = q;
+    long slot = 0;
+    for (int s : order) {
+        const int f0 = c.h_seg_faces[s], F = c.h_seg_faces[s + 1] - f0;
+        int G, fpw;
+        split(F, G, fpw);
+        segs[s] = int2{(int)slot, G};
+        slot += (long)GROUP_REP * GROUP_ROT * GROUP_ND * G;
+        for (int q = 0; q < G; q++)
+            tasks.push_back(GroupTask{s, q, f0 + q * fpw, std::min(f0 + F, f0 + (q + 1) * fpw)});
+    }
+    gp.threads = bs;
+    gp.width = width;
+    gp.total = (int)tasks.size();
+    gp.nslots = (int)slot;
+    gp.task.alloc(tasks.size());
+    gp.face.alloc(c.F);
+    gp.pos.alloc(c.F);
+    MHFEM_HIP(hipMemcpy(gp.face.p, face.data(), c.F * sizeof(int), hipMemcpyHostToDevice));
+    MHFEM_HIP(hipMemcpy(gp.pos.p, pos.data(), c.F * sizeof(int), hipMemcpyHostToDevice));
+    gp.seg.alloc(2 * (size_t)nseg);
+    MHFEM_HIP(hipMemcpy(gp.task.p, tasks.data(), tasks.size() * sizeof(GroupTask), hipMemcpyHostToDevice));
+    MHFEM_HIP(hipMemcpy(gp.seg.p, segs.data(), segs.size() * sizeof(int2), hipMemcpyHostToDevice));
+    gp.slots.alloc(slot);
+    gp.counters.alloc(2);
+    gp.pub.alloc((size_t)GROUP_ROT * c.rows * (fp32 ? 4 : 8));
+    return true;
+}
+
+template <typename T>
+void group_iterate(Ctx &c, GroupPlan &gp, const SellView<T> &A, double *sc, T *x, T *r, T *p, const T *r_ast)
+{
+    const int64_t pubn = (int64_t)GROUP_ROT * c.rows;
+    T *pub = reinterpret_cast<T *>(gp.pub.p);
+    int *ticket = gp.counters.p;
+    unsigned *beat = reinterpret_cast<unsigned *>(gp.counters.p + 1);
+    const unsigned g = (unsigned)std::min<int64_t>(1024, (std::max<int64_t>(pubn, gp.nslots) + 255) / 256);
+    hipLaunchKernelGGL(k_group_prepare<T>, g, 256, 0, c.stream, pubn, pub, gp.nslots, gp.slots.p, ticket, beat);
+    const GroupView v{gp.total, c.rows, gp.task.p, gp.face.p, gp.pos.p, reinterpret_cast<const int2 *>(gp.seg.p), ticket, beat, gp.slots.p,
+                      sc, gp.wait_ticks};
+    with_threads<T>(gp.threads, c.n, gp.width, [&](auto NC, auto WC, auto BC) {
+        constexpr int BS = decltype(BC)::value;
+        hipLaunchKernelGGL((k_bicg_group<T, decltype(NC)::value, decltype(WC)::value, BS, holds(sizeof(T), decltype(NC)::value, decltype(WC)::value)>), gp.total, BS, 0, c.stream, A,
+                           v, x, r, p, r_ast, pub);
+    });
+    MHFEM_HIP(hipGetLastError());
+}
+template void group_iterate<double>(Ctx &, GroupPlan &, const SellView<double> &, double *, double *, double *, double *,
+                                    const double *);
+template void group_iterate<float>(Ctx &, GroupPlan &, const SellView<float> &, double *, float *, float *, float *,
+                                   const float *);
+
+void group_clear_failed(Ctx &c, double *sc, int nseg)
+{
+    hipLaunchKernelGGL(k_group_failed, (nseg + 63) / 64, 64, 0, c.stream, sc, nseg);
+    MHFEM_HIP(hipGetLastError());
+}
+
+}  // namespace mhfem

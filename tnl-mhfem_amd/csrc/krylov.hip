@@ -31,6 +31,7 @@
 #include <unordered_map>
 
 #include "common.hpp"
+#include "device.hpp"
 
 namespace mhfem {
 
@@ -62,13 +63,6 @@ __device__ __forceinline__ bool seg_selected(const double *sc, int mode)
     if (mode == M_ACTIVE) return !halted(sc);
     if (mode == M_RESTART) return sc[S_RESTART] != 0.0;
     return true;
-}
-
-__device__ __forceinline__ double wave_sum(double v)
-{
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
-    return v;
 }
 
 __device__ void finalize(double *sc, int fin)
@@ -1151,49 +1145,6 @@ constexpr int ilu_lds_values()
     return ILU_WG * N + ILU_IMPORTS + pad;
 }
 
-template <typename T>
-struct SentinelBits;
-template <>
-struct SentinelBits<double> {
-    using U = unsigned long long;
-    static constexpr U bits = 0x7FF4A5A5A5A5A5A5ull;
-};
-template <>
-struct SentinelBits<float> {
-    using U = unsigned int;
-    static constexpr U bits = 0x7FA5A5A5u;
-};
-template <typename T>
-__device__ __forceinline__ bool is_sentinel(T v)
-{
-    return __builtin_bit_cast(typename SentinelBits<T>::U, v) == SentinelBits<T>::bits;
-}
-template <typename T>
-__device__ __forceinline__ T sentinel_value()
-{
-    return __builtin_bit_cast(T, SentinelBits<T>::bits);
-}
-template <typename T>
-__device__ __forceinline__ T coherent_load(const T *p)
-{
-    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-template <typename T>
-__device__ __forceinline__ void coherent_store(T *p, T v)
-{
-    __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-template <typename T>
-__device__ __forceinline__ T lds_load(const T *p)
-{
-    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-}
-template <typename T>
-__device__ __forceinline__ void lds_store(T *p, T v)
-{
-    __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-}
-
 struct IluSweep {
     int faces, nchunks;
     const int *rp, *dg;
@@ -1679,6 +1630,8 @@ struct Krylov {
     DBuf<int> perm, iperm, slice_width32, col32;
     DBuf<int64_t> slice_ptr32, map32;
     int64_t blocks32 = 0, diag_base32 = 0;
+    // BiCGStab of systems that fit on the chip, one launch per solve (group.hip)
+    GroupPlan group;
     // GMRES
     DBuf<double> V;
     int V_m = 0;
@@ -1691,6 +1644,7 @@ struct Krylov {
     hipGraphExec_t g_first = nullptr, g_more = nullptr, g_post = nullptr;
     double g_tau = 0;
     int g_iters = 0;
+    bool g_grouped = false;  // captured without iterations
     SchemeView g_view{};
     hipStream_t g_stream = nullptr;
 };
@@ -2373,6 +2327,12 @@ Krylov *krylov_create(Ctx &c)
                                &k->As32, &k->tmp32, &k->rhs32})
             b->alloc(n);
     }
+    if (c.cfg.solver == MHFEM_SOLVER_BICGSTAB && c.unit_diagonal &&
+        (c.cfg.preconditioner == MHFEM_PREC_DIAGONAL || c.cfg.preconditioner == MHFEM_PREC_NONE)) {
+        int width = 0;
+        for (int E = 0; E < c.F; E++) width = std::max<int>(width, (int)(c.h_bptr[E + 1] - c.h_bptr[E]));
+        group_plan(c, k->group, c.cfg.precision != MHFEM_PRECISION_FP64, width);
+    }
     return k;
 }
 
@@ -2617,6 +2577,15 @@ struct Solve {
         return sizeof(T) == 4 && !separate_prec();
     }
 
+    // the iteration in precision T runs in one launch (group.hip); timing
+    // level 2 samples the launches of the product, so it keeps those
+    template <typename T>
+    bool grouped() const
+    {
+        return k.group.total > 0 && k.group.cooldown == 0 && c.timing_level < 2 && !separate_prec() &&
+               !jacobi_scales() && (sizeof(T) == 4) == (c.cfg.precision != MHFEM_PRECISION_FP64);
+    }
+
     // The assembled MHFEM rows are scaled so that every diagonal entry is
     // exactly 1 (LinearSystem.h:196-201, BoundaryConditions.hpp:200-203,
     // :375-377): the diagonal preconditioner is then the identity and its
@@ -2819,6 +2788,24 @@ struct Solve {
     // once) and short solves would lose more than they gain.
     int bicg_drive(const T *b, T *x, const Vecs &v, More &&more)
     {
+        if (grouped<T>()) {
+            // every segment iterates inside one launch; the host restarts
+            // segments that broke down, and takes the launched iteration
+            // below when a wait in the kernel gave up
+            for (;;) {
+                group_iterate<T>(c, k.group, matrix<T>(), k.sc.p, x, (T *)v.r, (T *)v.p, (const T *)v.r_ast);
+                poll();
+                bool failed = false;
+                for (int s = 0; s < k.nseg; s++) failed |= seg_sc(s)[S_FAIL] != 0.0;
+                if (failed) {
+                    k.group.cooldown = 8;
+                    group_clear_failed(c, k.sc.p, k.nseg);
+                    break;
+                }
+                if (all_done()) return most_iterations();
+                bicg_init<T>(b, x, v, M_RESTART);
+            }
+        }
         Narrowed narrowed(*this);
         const size_t bytes = (size_t)k.nseg * NSLOTS * sizeof(double);
         auto snap = [&](int q) {
@@ -2874,6 +2861,10 @@ struct Solve {
             narrowed.synchronized();
             narrowed.update();
         }
+        return most_iterations();
+    }
+    int most_iterations() const
+    {
         int it = 0;
         for (int s = 0; s < k.nseg; s++) it = std::max(it, (int)seg_sc(s)[S_IT]);
         return it;
@@ -3638,6 +3629,8 @@ static void precond_update(Ctx &c, Krylov &k)
 
 Amg *krylov_amg(const Krylov &k) { return k.amg; }
 
+void krylov_set_group_wait(Krylov &k, unsigned long long ticks) { k.group.wait_ticks = ticks; }
+
 bool krylov_isai_info(const Krylov &k, long *nnz_lower, long *nnz_upper, int *rebuilds)
 {
     if (!k.isai.lo.rp.p) return false;
@@ -3841,6 +3834,7 @@ void krylov_solve(Ctx &c, const double *b, double *x, mhfem_solve_stats *st)
     if (c.timing) MHFEM_HIP(hipEventRecord(e1, c.stream));
     const double tol = c.cfg.convergence_residue;
     const int maxit = c.cfg.max_iterations;
+    if (k.group.cooldown > 0) k.group.cooldown--;
     mhfem_solve_stats out{};
     if (c.guess && c.guess_on_solve) guess_before_solve(c, *c.guess, b, x);
     if (k.nseg > 1 && (c.cfg.solver != MHFEM_SOLVER_BICGSTAB || c.cfg.precision != MHFEM_PRECISION_FP64))
@@ -4084,9 +4078,11 @@ void krylov_graph_step(Ctx &c, double time, double tau, mhfem_solve_stats *st)
     // boundary model switched on) re-captures them.  SchemeView is built
     // zero-initialised, so its padding compares equal.
     const SchemeView view = c.view();
-    if (k.g_first && (k.g_tau != tau || k.g_iters != every || std::memcmp(&k.g_view, &view, sizeof view) != 0))
-        drop_graphs(k);
+    if (k.group.cooldown > 0) k.group.cooldown--;
     Solve S(c, k);
+    const bool grouped = S.grouped<double>();
+    if (k.g_first && (k.g_tau != tau || k.g_iters != every || k.g_grouped != grouped || std::memcmp(&k.g_view, &view, sizeof view) != 0))
+        drop_graphs(k);
     Solve::Vecs v{k.r.p, k.r_ast.p, k.p.p, k.Ap.p, k.s.p, k.As.p, k.tmp.p, k.tmp2.p, k.dinv.p};
     const double *b = c.arr[MHFEM_RHS].p;
     double *x = c.arr[MHFEM_Z_iF].p;
@@ -4107,12 +4103,13 @@ void krylov_graph_step(Ctx &c, double time, double tau, mhfem_solve_stats *st)
             launch_assemble(c, time, tau);
             precond_update(c, k);
             S.bicg_start<double>(b, x, v, c.cfg.convergence_residue, c.cfg.max_iterations);
-            S.bicg_iterations<double>(x, v, every);
+            if (!grouped) S.bicg_iterations<double>(x, v, every);
         }, &k.g_first);
         capture([&]() { S.bicg_iterations<double>(x, v, every); }, &k.g_more);
         capture([&]() { launch_post_iterate(c); }, &k.g_post);
         k.g_tau = tau;
         k.g_iters = every;
+        k.g_grouped = grouped;
         k.g_view = view;
         k.g_stream = c.stream;
     }
