@@ -1651,6 +1651,22 @@ struct Krylov {
 
 static inline unsigned grid_for(long n) { return (unsigned)std::max<long>(1, std::min<long>((n + KB - 1) / KB, MAXG)); }
 
+// Rows per work-group when the caller names none: about 1500 work-groups, so
+// that small systems still fill the CUs (with 2048 rows 169,000 unknowns made
+// 83 work-groups), within 512 and 2048 rows (more partial sums cost the
+// reductions more than smaller work-groups gain).  Measured, us per iteration
+// with 512 / 1024 / 2048 rows: 669,000 unknowns FP64 n = 2 64.3 / 64.1 / 75.9;
+// 777,000 FP64 n = 1 58.8 / 63.1 / 85.8; 972,000 FP32 n = 2 56.5 / 55.9 /
+// 61.0; 2.7 M FP64 n = 2 229 / 231 / 238; 6.3 M FP32 n = 2 265 / 262 / 260;
+// ILU(0) on 169,000 771 / 782 / 808; GMRES on 197,000 115 / 117 / 124.  256
+// rows were slower from 669,000 unknowns on and no faster below.
+static int default_rows(int rows)
+{
+    int rpb = 512;
+    while (rpb < 2048 && rows / 1500 >= 2 * rpb) rpb *= 2;
+    return rpb;
+}
+
 // work-group tables for `rpb` rows per work-group, segment aligned
 static void build_blocks(Ctx &c, Krylov &k, int rpb)
 {
@@ -2282,7 +2298,7 @@ Krylov *krylov_create(Ctx &c)
                                 hipHostMallocDefault));
         MHFEM_HIP(hipEventCreateWithFlags(&k->ev_ahead[q], hipEventDisableTiming));
     }
-    build_blocks(c, *k, c.cfg.rows_per_block > 0 ? c.cfg.rows_per_block : 2048);
+    build_blocks(c, *k, c.cfg.rows_per_block > 0 ? c.cfg.rows_per_block : default_rows(n));
     if (c.cfg.preconditioner == MHFEM_PREC_ILUT) k->ilu.a0.alloc(c.nnz);
     // level tables: ILU(0), the ISAI factors and SOR's sweeps
     if (c.cfg.preconditioner == MHFEM_PREC_ILU0 || is_isai(c.cfg.preconditioner) || c.cfg.solver == MHFEM_SOLVER_SOR) {
