@@ -64,13 +64,25 @@ def test_one_launch_matches_oracle(case, precision, groups):
     s.close()
 
 
-@pytest.mark.parametrize("precision", ["fp64", "fp32-reliable"])
-def test_a_wait_that_gives_up_hands_over(precision):
+@pytest.mark.parametrize("restart", [3, 30, 32])
+@pytest.mark.parametrize("case", sorted(CASES))
+def test_gmres_cycles_match_oracle(case, restart):
+    """GMRES(m) with each cycle in one launch; restarts of 3 (a part of a
+    group of four dot products), 30 (the default) and 32 (the largest)."""
+    print(f"\n[group] gmres {case} m {restart}", flush=True)
+    pr = CASES[case]()
+    s = capi.Solver(pr, solver="gmres", preconditioner="diagonal", tol=1e-13, gmres_restart=restart)
+    _steps(pr, s, pyoracle.Oracle(pr))
+    s.close()
+
+
+@pytest.mark.parametrize("solver,precision", [("bicgstab", "fp64"), ("bicgstab", "fp32-reliable"), ("gmres", "fp64")])
+def test_a_wait_that_gives_up_hands_over(solver, precision):
     """With a bound of zero the first wait between two work-groups gives up:
     the solve is finished by the launched iteration, and so are the next ones."""
     pr = problems.adr_3d(s=6, n=2, preconditioner="diagonal")
-    print(f"\n[group] handed over, {precision}", flush=True)
-    s = capi.Solver(pr, preconditioner="diagonal", tol=1e-13, precision=precision, inner_tol=0.03)
+    print(f"\n[group] handed over, {solver} {precision}", flush=True)
+    s = capi.Solver(pr, solver=solver, preconditioner="diagonal", tol=1e-13, precision=precision, inner_tol=0.03)
     fn = capi.lib().mhfem_internal_group_wait
     fn.argtypes = [C.c_void_p, C.c_ulonglong]
     assert fn(s.ctx, 0) == 0

@@ -380,7 +380,11 @@ struct GroupPlan {
     int cooldown = 0;    // solves left that iterate by launches after a wait gave up
     unsigned long long wait_ticks = 500000;  // 5 ms of the 100 MHz counter without any iteration in the launch
 };
-bool group_plan(Ctx &c, GroupPlan &gp, bool fp32, int width);
+bool group_plan(Ctx &c, GroupPlan &gp, bool fp32, int width, bool gmres);
+// one cycle of GMRES(m) from the residual r (norm beta), m <= group_gmres_restart()
+int group_gmres_restart();
+void group_gmres_cycle(Ctx &c, GroupPlan &gp, const SellView<double> &A, double *sc, const double *r, double *x,
+                       double *V, int m, double beta, double bnorm, double tol, int it, int maxit);
 template <typename T>
 void group_iterate(Ctx &c, GroupPlan &gp, const SellView<T> &A, double *sc, T *x, T *r, T *p, const T *r_ast);
 void group_clear_failed(Ctx &c, double *sc, int nseg);

@@ -2343,11 +2343,13 @@ Krylov *krylov_create(Ctx &c)
                                &k->As32, &k->tmp32, &k->rhs32})
             b->alloc(n);
     }
-    if (c.cfg.solver == MHFEM_SOLVER_BICGSTAB && c.unit_diagonal &&
+    const bool gmres = c.cfg.solver == MHFEM_SOLVER_GMRES && k->nseg == 1 &&
+                       c.cfg.gmres_restart <= group_gmres_restart();
+    if ((c.cfg.solver == MHFEM_SOLVER_BICGSTAB || gmres) && c.unit_diagonal &&
         (c.cfg.preconditioner == MHFEM_PREC_DIAGONAL || c.cfg.preconditioner == MHFEM_PREC_NONE)) {
         int width = 0;
         for (int E = 0; E < c.F; E++) width = std::max<int>(width, (int)(c.h_bptr[E + 1] - c.h_bptr[E]));
-        group_plan(c, k->group, c.cfg.precision != MHFEM_PRECISION_FP64, width);
+        group_plan(c, k->group, c.cfg.precision != MHFEM_PRECISION_FP64, width, gmres);
     }
     return k;
 }
@@ -3002,6 +3004,23 @@ int Solve::gmres(const double *b, double *x, double tol, int maxit, int m, doubl
     DBuf<double> gpart;  // partial dots of the Gram-Schmidt step: (m+1) rows of gg
     gpart.alloc((size_t)(m + 1) * gg);
     while (resid >= tol && it < maxit && !std::isnan(resid)) {
+        if (grouped<double>() && beta > 0.0) {
+            // the cycle in one launch; V's first vector is the residual until then
+            copy(V, k.r.p);
+            group_gmres_cycle(c, k.group, matrix<double>(), k.sc.p, k.r.p, x, V, m, beta, b_norm, tol, it, maxit);
+            presidue<double>(x, b, V, tmp, dinv, M_ALL);
+            const double norm = norm2(V);
+            if (k.h_sc[S_FAIL] != 0.0) {
+                k.group.cooldown = 8;  // this solve and the next go on with launches
+                hipLaunchKernelGGL(k_set_slot, 1, 64, 0, c.stream, k.sc.p, (int)S_FAIL, 0.0);
+                MHFEM_HIP(hipGetLastError());
+            } else {
+                it = (int)k.h_sc[S_IT];
+            }
+            beta = norm;
+            resid = beta / b_norm;
+            continue;
+        }
         hipLaunchKernelGGL(k_scale_into, g, KB, 0, c.stream, n, V, 1.0 / beta, V);
         std::fill(gv.begin(), gv.end(), 0.0);
         gv[0] = beta;
