@@ -33,17 +33,14 @@
 //   from the iterate it has (and keeps to that for the next solves).
 //
 // Measured (MI355X, whole trajectories as in perf/cases.py, launched -> one
-// launch): 64 x 64 x 2 triangles, 3 steps 3.21 -> 0.59 ms; 201 x 201 x 2,
-// 2 steps 6.37 -> 1.50 ms; 21^3 x 6 tetrahedra n = 1, 2 steps 17.7 -> 2.71 ms
-// (48 -> 7.2 us per iteration); 20^3 x 6 n = 2, FP32, 6 steps 50.5 -> 13.1 ms;
-// 20^3 voxels n = 3, 6.77 -> 1.93 ms; 32 ragged 2-D instances 40.8 -> 20.4 ms.
-// An exchange takes 3.0-3.7 us with 200 work-groups (2 us with 25): 0.5 us of
-// arithmetic, 0.4 us of work-group sums, 2 us from the post of the slowest
-// work-group to its sum in every other one.  Tried: neighbours polled only
-// after the sums are in (10 us per iteration instead of 8); wavefronts that
-// sleep before they poll (no change); the partial sums in one copy instead of
-// GROUP_REP (5 % slower at 200 work-groups); faces in the mesh order (gathers
-// 2.3 us instead of 1.6).
+// launch): 64 x 64 x 2 triangles, 3 steps 3.21 -> 0.55 ms; 201 x 201 x 2,
+// 2 steps 6.37 -> 1.05 ms; 21^3 x 6 tetrahedra n = 1, 2 steps 17.7 -> 1.94 ms
+// (48 -> 4.9 us per iteration); 20^3 x 6 n = 2, FP32, 6 steps 50.5 -> 10.3 ms;
+// 32 ragged 2-D instances 40.8 -> 13.2 ms.  An exchange takes 2.4 us with 200
+// work-groups: 0.5 us of arithmetic, 0.4 us of work-group sums, the rest from
+// the post of the slowest work-group to its sum in every other one.  Tried:
+// neighbours polled only after the sums are in (10 us per iteration where 8
+// were needed then); faces in the mesh order (gathers 2.3 us instead of 1.6).
 #include <algorithm>
 #include <type_traits>
 
@@ -54,6 +51,14 @@ namespace mhfem {
 
 constexpr int GROUP_ROT = 4;  // rotating copies of the published vectors and partial sums
 constexpr int GROUP_REP = 8;  // copies of the partial sums, each read by every 8th work-group
+// Pause before the first look at the others' values, in 64 cycles (0.48 us at
+// 2.4 GHz).  They cannot be there sooner than a store and a load take, and
+// looks before that only load the fabric that carries them: us per iteration
+// with 0 / 12 / 16 / 20 / 24 / 40: 114,000 faces 7.1 / 5.7 / 4.9 / 5.1 / 5.3 /
+// 6.1; the 32 ragged instances 18.0 / 14.9 / 13.9 / 12.5 / 12.8 / 14.6 ms; 12,400
+// faces 6.4 / 6.2 / 6.1 / 6.3 / 6.5 / 7.4.  Later looks gain nothing from longer
+// pauses (4 or 8 instead of 1: 2-20 % slower).
+constexpr int GROUP_FIRST_LOOK = 18;
 constexpr int GROUP_ND = 4;   // dot products of a reduction, at most
 
 // partial sums a wavefront adds, per dot product: BS / 256 wavefronts for each
@@ -314,6 +319,7 @@ __global__ void __launch_bounds__(BS) k_bicg_group(SellView<T> A, GroupView g, T
             v[q] = 0.0;
             if (chunk + q * 64 + lane < G) pd |= 1u << q;
         }
+        __builtin_amdgcn_s_sleep(GROUP_FIRST_LOOK);
         for (;;) {
 #pragma unroll
             for (int k = 0; k < W; k++)
@@ -492,7 +498,7 @@ __global__ void __launch_bounds__(BS) k_bicg_group(SellView<T> A, GroupView g, T
 // Givens rotations are done by one lane of every work-group, the same numbers
 // in each.  The launched form takes ten launches and three host reads per
 // iteration.  Measured at 197,000 unknowns (20^3 x 6 tetrahedra, n = 2,
-// m = 30): 118 -> 28 us per iteration, the step 49.9 -> 11.4 ms; about 11 us of
+// m = 30): 118 -> 24 us per iteration, the step 49.9 -> 9.7 ms; about 8 us of
 // an iteration are the three exchanges, the rest the four passes over V and
 // the rotations.
 constexpr int GMRES_M = 32;
@@ -615,6 +621,7 @@ __global__ void __launch_bounds__(BS) k_gmres_group(SellView<double> A, GroupVie
                 s4[d][q] = 0.0;
                 if (wid + NW * d < nd && q * 64 + lane < G) pd |= 1u << (d * SL + q);
             }
+        __builtin_amdgcn_s_sleep(GROUP_FIRST_LOOK);
         for (;;) {
             if constexpr (PUB) {
 #pragma unroll
