@@ -27,7 +27,7 @@ void set_global_error(const std::string &msg);
 // device scalar slots of the Krylov solver (per segment)
 enum Slot {
     S_RHO = 0, S_RHO_OLD, S_ALPHA, S_OMEGA, S_BETA, S_RAST_SQ, S_BNORM, S_RESID, S_TOL, S_IT,
-    S_DONE, S_RESTART, S_MAXIT, S_D0, S_D1, S_D2, S_D3, S_TOLABS, S_DELTA, S_BFIX, S_BREAK, S_FAIL, NSLOTS = 32
+    S_DONE, S_RESTART, S_MAXIT, S_D0, S_D1, S_D2, S_D3, S_TOLABS, S_DELTA, S_BFIX, S_BREAK, S_FAIL, S_LIMIT, S_BROKEN, S_BN0, S_TOL0, NSLOTS = 32
 };
 // a segment's solve has stopped (converged, failed or waiting for a restart):
 // kernels queued behind it return at once
@@ -385,8 +385,9 @@ bool group_plan(Ctx &c, GroupPlan &gp, bool fp32, int width, bool gmres);
 int group_gmres_restart();
 void group_gmres_cycle(Ctx &c, GroupPlan &gp, const SellView<double> &A, double *sc, const double *r, double *x,
                        double *V, int m, double beta, double bnorm, double tol, int it, int maxit);
+// q: the direction starts as r + S_BFIX q instead of p
 template <typename T>
-void group_iterate(Ctx &c, GroupPlan &gp, const SellView<T> &A, double *sc, T *x, T *r, T *p, const T *r_ast);
+void group_iterate(Ctx &c, GroupPlan &gp, const SellView<T> &A, double *sc, T *x, T *r, T *p, const T *r_ast, const T *q);
 void group_clear_failed(Ctx &c, double *sc, int nseg);
 void krylov_set_group_wait(Krylov &k, unsigned long long ticks);
 

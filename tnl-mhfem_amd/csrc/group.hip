@@ -173,7 +173,8 @@ struct GroupWait {
 
 template <typename T, int N, int W, int BS, bool HOLD>
 __global__ void __launch_bounds__(BS) k_bicg_group(SellView<T> A, GroupView g, T *__restrict__ xg, T *__restrict__ rg,
-                                                   T *__restrict__ pg, const T *__restrict__ r_ast, T *pub)
+                                                   T *__restrict__ pg, const T *__restrict__ r_ast,
+                                                   const T *__restrict__ qg, T *pub)
 {
     constexpr int NW = BS / 64, SLOTS = group_slots(BS);
     __shared__ int s_ticket, s_fail;
@@ -215,6 +216,16 @@ __global__ void __launch_bounds__(BS) k_bicg_group(SellView<T> A, GroupView g, T
         base = A.slice_ptr[f >> 6] + (f & 63);
         w = A.slice_width[f >> 6];
     }
+    // the direction after a reliable update: r + S_BFIX q
+    const T fix = qg ? (T)uniform(sc[S_BFIX]) : T(0);
+    auto direction = [&](int face, const Pack<T, N> &res) {
+        Pack<T, N> d = ld<T, N>((qg ? qg : pg) + (int64_t)face * N);
+        if (qg) {
+#pragma unroll
+            for (int i = 0; i < N; i++) d.v[i] = res.v[i] + fix * d.v[i];
+        }
+        return d;
+    };
     unsigned remote = 0;  // neighbours in other work-groups
     bool alone = true;    // no neighbour but itself (padding)
 #pragma unroll
@@ -228,8 +239,8 @@ __global__ void __launch_bounds__(BS) k_bicg_group(SellView<T> A, GroupView g, T
         for (int i = 0; i < N; i++) pn[k].v[i] = rn[k].v[i] = T(0);
         if (k < w) {
             if constexpr (HOLD) val[k] = ld<T, N * N>(A.val + (base + (int64_t)k * 64) * (N * N));
-            pn[k] = ld<T, N>(pg + (int64_t)col[k] * N);
             rn[k] = ld<T, N>(rg + (int64_t)col[k] * N);
+            pn[k] = direction(col[k], rn[k]);
         }
         alone = alone && col[k] == f;
         col[k] = k < w ? g.pos[col[k]] : task.p0;
@@ -242,8 +253,8 @@ __global__ void __launch_bounds__(BS) k_bicg_group(SellView<T> A, GroupView g, T
     const bool shared_face = valid && (remote != 0 || alone);
     own[0][tid] = own[1][tid] = p;
     if (valid) {
-        p = ld<T, N>(pg + (int64_t)f * N);
         r = ld<T, N>(rg + (int64_t)f * N);
+        p = direction(f, r);
         own[0][tid] = ld<T, N>(xg + (int64_t)f * N);
         own[1][tid] = ld<T, N>(r_ast + (int64_t)f * N);
         if constexpr (N > 1) dg = ld<T, N *(N - 1)>(A.val + A.diag_base + (int64_t)f * N * (N - 1));
@@ -1017,7 +1028,8 @@ bool group_plan(Ctx &c, GroupPlan &gp, bool fp32, int width, bool gmres)
 }
 
 template <typename T>
-void group_iterate(Ctx &c, GroupPlan &gp, const SellView<T> &A, double *sc, T *x, T *r, T *p, const T *r_ast)
+void group_iterate(Ctx &c, GroupPlan &gp, const SellView<T> &A, double *sc, T *x, T *r, T *p, const T *r_ast,
+                   const T *q)
 {
     const int64_t pubn = (int64_t)GROUP_ROT * c.rows;
     T *pub = reinterpret_cast<T *>(gp.pub.p);
@@ -1030,14 +1042,14 @@ void group_iterate(Ctx &c, GroupPlan &gp, const SellView<T> &A, double *sc, T *x
     with_threads<T>(gp.threads, c.n, gp.width, [&](auto NC, auto WC, auto BC) {
         constexpr int BS = decltype(BC)::value;
         hipLaunchKernelGGL((k_bicg_group<T, decltype(NC)::value, decltype(WC)::value, BS, holds(sizeof(T), decltype(NC)::value, decltype(WC)::value)>), gp.total, BS, 0, c.stream, A,
-                           v, x, r, p, r_ast, pub);
+                           v, x, r, p, r_ast, q, pub);
     });
     MHFEM_HIP(hipGetLastError());
 }
 template void group_iterate<double>(Ctx &, GroupPlan &, const SellView<double> &, double *, double *, double *, double *,
-                                    const double *);
+                                    const double *, const double *);
 template void group_iterate<float>(Ctx &, GroupPlan &, const SellView<float> &, double *, float *, float *, float *,
-                                   const float *);
+                                   const float *, const float *);
 
 int group_gmres_restart() { return GMRES_M; }
 

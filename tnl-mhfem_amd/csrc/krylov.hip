@@ -39,9 +39,13 @@ constexpr int KB = 256;
 constexpr int MAXG = 2048;
 
 enum Fin { FIN_NONE = 0, FIN_ALPHA, FIN_OMEGA, FIN_UPDATE, FIN_BNORM, FIN_INIT, FIN_REPLACE,
-           FIN_ALPHA_MERGED, FIN_OMEGA_MERGED, FIN_REPLACE_MERGED };
+           FIN_ALPHA_MERGED, FIN_OMEGA_MERGED, FIN_REPLACE_MERGED, FIN_START };
 // which segments a kernel works on
 enum Mode { M_ALL = 0, M_ACTIVE = 1, M_RESTART = 2 };
+
+// iterations between two FP64 residual replacements, at most, so that a
+// recurrence that cannot reach the next one still reaches the stall test
+constexpr int ROUND_CAP = 300;
 
 // Segmented work decomposition.  Work-group b covers rows
 // [blk_row[b], blk_row[b+1]) of segment blk_seg[b]; segment s owns the
@@ -104,6 +108,12 @@ __device__ void finalize(double *sc, int fin)
         const double bn = sqrt(sc[S_D0]);
         sc[S_BNORM] = bn == 0.0 ? 1.0 : bn;
         break;
+    }
+    // D0 = (r, r), D2 = (b, b) of a start in one kernel (k_bicg_start)
+    case FIN_START: {
+        const double bn = sqrt(sc[S_D2]);
+        sc[S_BNORM] = bn == 0.0 ? 1.0 : bn;
+        [[fallthrough]];
     }
     case FIN_INIT: {
         sc[S_BREAK] = 0;
@@ -187,6 +197,11 @@ __device__ void finalize(double *sc, int fin)
     case FIN_REPLACE_MERGED: {
         const double rn = sqrt(sc[S_D0]);
         const double beta_old = sc[S_BETA];
+        // a round that ended in a breakdown, or gave up (group.hip), starts
+        // afresh from the replaced residual; one whose recurrence broke was
+        // not added to the solution (k_mixed_flush) and ends the FP32 solve
+        const bool again = sc[S_RESTART] != 0.0 || sc[S_FAIL] != 0.0;
+        if (!isfinite(sc[S_RESID])) sc[S_BROKEN] = 1;
         sc[S_RHO] = sc[S_D2];
         sc[S_BETA] = (sc[S_RHO] / sc[S_RHO_OLD]) * (sc[S_ALPHA] / sc[S_OMEGA]);
         const double fix = sc[S_BETA] / beta_old;
@@ -195,8 +210,11 @@ __device__ void finalize(double *sc, int fin)
         sc[S_BNORM] = rn;
         sc[S_TOL] = rn > 0 ? fmax(sc[S_DELTA], sc[S_TOLABS] / rn) : 1.0;
         sc[S_RESID] = 1.0;
-        sc[S_DONE] = rn == 0.0 ? 1 : 0;
-        sc[S_RESTART] = (rn > 0.0 && !(fabs(sc[S_RHO]) >= eps2 * sc[S_RAST_SQ])) ? 1 : 0;
+        // the round ends here as the host will decide (its test on the FP64
+        // residual), so that a round queued behind it returns at once
+        sc[S_DONE] = (!(rn / sc[S_BN0] >= sc[S_TOL0]) || sc[S_IT] >= sc[S_LIMIT] || sc[S_BROKEN] != 0.0) ? 1 : 0;
+        sc[S_RESTART] = (rn > 0.0 && (again || !(fabs(sc[S_RHO]) >= eps2 * sc[S_RAST_SQ]))) ? 1 : 0;
+        sc[S_MAXIT] = fmin(sc[S_LIMIT], sc[S_IT] + ROUND_CAP);
         break;
     }
     default: break;
@@ -537,6 +555,127 @@ __global__ void __launch_bounds__(KB) k_scopy2(Seg sg, int mode, const T *__rest
     }
 }
 
+// Start of a solve whose preconditioner is the identity on the unit-diagonal
+// rows: r = b - A x, p = r* = r and the partial sums (r, r), (r, r) (row 1,
+// read with the first merged alpha) and (b, b), where separate kernels copied
+// b and r twice and reduced twice.
+template <typename T, int N>
+__global__ void __launch_bounds__(KB) k_bicg_start(SellView<T> A, Seg sg, const T *__restrict__ x,
+                                                   const T *__restrict__ b, T *__restrict__ r, T *__restrict__ p,
+                                                   T *__restrict__ r_ast)
+{
+    SEG_BLOCK_PROLOGUE(sg, M_ALL);
+    double acc[3] = {0, 0, 0};
+    for (int f = row0_ / N + threadIdx.x; f < row1_ / N; f += KB) {
+        Pack<T, N> v = sell_face<N>(A, x, f);
+        const Pack<T, N> bb = ld<T, N>(b + (int64_t)f * N);
+#pragma unroll
+        for (int i = 0; i < N; i++) {
+            v.v[i] = bb.v[i] - v.v[i];
+            acc[0] += (double)v.v[i] * (double)v.v[i];
+            acc[2] += (double)bb.v[i] * (double)bb.v[i];
+        }
+        st<T, N>(r + (int64_t)f * N, v);
+        st<T, N>(p + (int64_t)f * N, v);
+        st<T, N>(r_ast + (int64_t)f * N, v);
+    }
+    acc[1] = acc[0];
+    block_partial<3>(acc, sg, blk_);
+}
+
+// The FP64 residual of the mixed-precision solve, rounded to FP32, in the
+// FP32 iteration's face order (iperm, identity if null): START writes r, p,
+// r* and the right-hand side of the FP32 system, clears its iterate and sums
+// (r, r), (r, r), (b, b); otherwise (a reliable update) r and the right-hand
+// side, and the sums (r, r), (r, r), (r, r*).
+template <int N, bool START>
+__global__ void __launch_bounds__(KB) k_mixed_residual(SellView<double> A, Seg sg, const double *__restrict__ x,
+                                                       const double *__restrict__ b, const int *__restrict__ iperm,
+                                                       float *__restrict__ r32, float *__restrict__ rhs32,
+                                                       float *__restrict__ p32, float *__restrict__ ra32,
+                                                       float *__restrict__ x32)
+{
+    SEG_BLOCK_PROLOGUE(sg, M_ALL);
+    double acc[3] = {0, 0, 0};
+    for (int f = row0_ / N + threadIdx.x; f < row1_ / N; f += KB) {
+        const Pack<double, N> v = sell_face<N>(A, x, f);
+        const Pack<double, N> bb = ld<double, N>(b + (int64_t)f * N);
+        const int64_t q = (int64_t)(iperm ? iperm[f] : f) * N;
+        Pack<float, N> r;
+#pragma unroll
+        for (int i = 0; i < N; i++) {
+            r.v[i] = (float)(bb.v[i] - v.v[i]);
+            acc[0] += (double)r.v[i] * (double)r.v[i];
+        }
+        st<float, N>(r32 + q, r);
+        st<float, N>(rhs32 + q, r);
+        if constexpr (START) {
+            Pack<float, N> zero;
+#pragma unroll
+            for (int i = 0; i < N; i++) {
+                zero.v[i] = 0.0f;
+                const double bf = (double)(float)bb.v[i];
+                acc[2] += bf * bf;
+            }
+            st<float, N>(p32 + q, r);
+            st<float, N>(ra32 + q, r);
+            st<float, N>(x32 + q, zero);
+        } else {
+            const Pack<float, N> ra = ld<float, N>(ra32 + q);
+#pragma unroll
+            for (int i = 0; i < N; i++) acc[2] += (double)r.v[i] * (double)ra.v[i];
+        }
+    }
+    acc[1] = acc[0];
+    block_partial<3>(acc, sg, blk_);
+}
+
+// Scalars of the FP32 recurrence after k_mixed_residual<START>
+__global__ void k_mixed_scalars(double *sc, double rr, double tol_inner, double delta, double bn0, double tol0,
+                                double limit)
+{
+    if (threadIdx.x != 0) return;
+    for (int k = 0; k < NSLOTS; k++) sc[k] = 0.0;
+    sc[S_BNORM] = sqrt(rr);
+    sc[S_RHO] = rr;
+    sc[S_RAST_SQ] = rr;
+    sc[S_RESID] = 1.0;
+    sc[S_TOL] = tol_inner;
+    sc[S_MAXIT] = fmin(limit, (double)ROUND_CAP);
+    sc[S_TOLABS] = tol0 * bn0;
+    sc[S_DELTA] = delta;
+    sc[S_LIMIT] = limit;
+    sc[S_BN0] = bn0;
+    sc[S_TOL0] = tol0;
+    sc[S_DONE] = (!(1.0 >= tol_inner) || 0.0 >= limit) ? 1 : 0;
+}
+
+// End of a round of the FP32 recurrence: x += d, d = 0 (skipped when the
+// recurrence broke down to non-finite numbers), q = p - r
+template <int N>
+__global__ void __launch_bounds__(KB) k_mixed_flush(int faces, const double *sc, const int *__restrict__ iperm,
+                                                    double *__restrict__ x, float *__restrict__ d,
+                                                    const float *__restrict__ p, const float *__restrict__ r,
+                                                    float *__restrict__ qv)
+{
+    const bool broken = !isfinite(sc[S_RESID]);
+    for (int f = blockIdx.x * KB + threadIdx.x; f < faces; f += gridDim.x * KB) {
+        const int64_t q = (int64_t)(iperm ? iperm[f] : f) * N;
+        Pack<double, N> xv = ld<double, N>(x + (int64_t)f * N);
+        const Pack<float, N> dv = ld<float, N>(d + q), pv = ld<float, N>(p + q), rv = ld<float, N>(r + q);
+        Pack<float, N> zero, dir;
+#pragma unroll
+        for (int i = 0; i < N; i++) {
+            xv.v[i] += broken ? 0.0 : (double)dv.v[i];
+            zero.v[i] = 0.0f;
+            dir.v[i] = pv.v[i] - rv.v[i];
+        }
+        st<double, N>(x + (int64_t)f * N, xv);
+        st<float, N>(d + q, zero);
+        st<float, N>(qv + q, dir);
+    }
+}
+
 // s = r - alpha Ap
 template <typename T>
 __global__ void __launch_bounds__(KB) k_bicg_s(Seg sg, const T *__restrict__ r, const T *__restrict__ Ap,
@@ -599,15 +738,8 @@ __global__ void __launch_bounds__(KB) k_bicg_xrp(Seg sg, T *__restrict__ x, T *_
     block_partial<1, 1>(acc, sg, blk_);
 }
 
-// merged iteration, after a reliable update: q = p - r (before r is
-// replaced), then p = r + S_BFIX q (after)
-template <typename T>
-__global__ void __launch_bounds__(KB) k_bicg_dir(Seg sg, const T *__restrict__ p, const T *__restrict__ r,
-                                                 T *__restrict__ q)
-{
-    SEG_BLOCK_PROLOGUE(sg, M_ALL);
-    for (int i = row0_ + threadIdx.x; i < row1_; i += KB) q[i] = p[i] - r[i];
-}
+// merged iteration, after a reliable update: p = r + S_BFIX q with q = p - r
+// of before it (k_mixed_flush)
 template <typename T>
 __global__ void __launch_bounds__(KB) k_bicg_pfix(Seg sg, const T *__restrict__ r, T *__restrict__ p,
                                                   const T *__restrict__ q)
@@ -2298,6 +2430,9 @@ Krylov *krylov_create(Ctx &c)
                                 hipHostMallocDefault));
         MHFEM_HIP(hipEventCreateWithFlags(&k->ev_ahead[q], hipEventDisableTiming));
     }
+    // the diagonal is 1 by construction: the Jacobi scaling is 1 / 1
+    hipLaunchKernelGGL((k_fill_t<double>), grid_for(n), KB, 0, c.stream, (long)n, k->dinv.p, 1.0);
+    MHFEM_HIP(hipGetLastError());
     build_blocks(c, *k, c.cfg.rows_per_block > 0 ? c.cfg.rows_per_block : default_rows(n));
     if (c.cfg.preconditioner == MHFEM_PREC_ILUT) k->ilu.a0.alloc(c.nnz);
     // level tables: ILU(0), the ISAI factors and SOR's sweeps
@@ -2342,6 +2477,8 @@ Krylov *krylov_create(Ctx &c)
         for (DBuf<float> *b : {&k->dinv32, &k->b32, &k->x32, &k->r32, &k->r_ast32, &k->p32, &k->Ap32, &k->s32,
                                &k->As32, &k->tmp32, &k->rhs32})
             b->alloc(n);
+        hipLaunchKernelGGL((k_fill_t<float>), grid_for(n), KB, 0, c.stream, (long)n, k->dinv32.p, 1.0f);
+        MHFEM_HIP(hipGetLastError());
     }
     const bool gmres = c.cfg.solver == MHFEM_SOLVER_GMRES && k->nseg == 1 &&
                        c.cfg.gmres_restart <= group_gmres_restart();
@@ -2595,7 +2732,7 @@ struct Solve {
     template <typename T>
     bool merged() const
     {
-        return !separate_prec();
+        return plain_prec();
     }
 
     // the iteration in precision T runs in one launch (group.hip); timing
@@ -2612,6 +2749,9 @@ struct Solve {
     // :375-377): the diagonal preconditioner is then the identity and its
     // scaling vector is not read.
     bool jacobi_scales() const { return c.cfg.preconditioner == MHFEM_PREC_DIAGONAL && !c.unit_diagonal; }
+
+    // no preconditioner, or the diagonal one on unit-diagonal rows: M = 1
+    bool plain_prec() const { return !separate_prec() && !jacobi_scales(); }
 
     // ---- preconditioner apply y = M^{-1} x (T = double or float)
     template <typename T>
@@ -2748,6 +2888,15 @@ struct Solve {
     void bicg_start(const T *b, T *x, const Vecs &v, double tol, int maxit)
     {
         set_scalars(tol, maxit);
+        if (plain_prec()) {
+            SellView<T> A = matrix<T>();
+            with_n(c.n, [&](auto NC) {
+                hipLaunchKernelGGL((k_bicg_start<T, decltype(NC)::value>), k.nblk, KB, 0, c.stream, A, seg(M_ALL),
+                                   (const T *)x, b, (T *)v.r, (T *)v.p, (T *)v.r_ast);
+            });
+            finish<3>(FIN_START, M_ALL);
+            return;
+        }
         prec<T>(b, (T *)v.tmp2, (const T *)v.dinv, M_ALL);
         dots<T, 1>(DotArgs<T, 1>{{(T *)v.tmp2}, {(T *)v.tmp2}}, FIN_BNORM, M_ALL);
         bicg_init<T>(b, x, v, M_ALL);
@@ -2814,7 +2963,8 @@ struct Solve {
             // segments that broke down, and takes the launched iteration
             // below when a wait in the kernel gave up
             for (;;) {
-                group_iterate<T>(c, k.group, matrix<T>(), k.sc.p, x, (T *)v.r, (T *)v.p, (const T *)v.r_ast);
+                group_iterate<T>(c, k.group, matrix<T>(), k.sc.p, x, (T *)v.r, (T *)v.p, (const T *)v.r_ast,
+                                 (const T *)nullptr);
                 poll();
                 bool failed = false;
                 for (int s = 0; s < k.nseg; s++) failed |= seg_sc(s)[S_FAIL] != 0.0;
@@ -2889,6 +3039,99 @@ struct Solve {
         int it = 0;
         for (int s = 0; s < k.nseg; s++) it = std::max(it, (int)seg_sc(s)[S_IT]);
         return it;
+    }
+
+    // One FP32 recurrence with reliable updates (Sleijpen & van der Vorst
+    // 1996), M = 1: each time its residual has dropped by inner_tol, the FP32
+    // correction goes into the FP64 solution, the FP64 residual replaces the
+    // recursive one and the recurrence goes on with its search direction and
+    // shadow residual.  A system that iterates in one launch queues the next
+    // round before the host has read the residual of the last: the device
+    // takes the same decisions (FIN_REPLACE_MERGED), and a round queued after
+    // the end returns at once.
+    void reliable(const double *b, double *x, const Vecs &v, double tol, int maxit, double inner_tol, int *total,
+                  int *outer, double *res, bool *fallback)
+    {
+        float *r = (float *)v.r, *p = (float *)v.p, *ra = (float *)v.r_ast, *q = (float *)v.s;
+        const int *iperm = k.permuted ? (const int *)k.iperm.p : (const int *)nullptr;
+        const SellView<double> A = matrix<double>();
+        auto residual = [&](auto START) {
+            with_n(c.n, [&](auto NC) {
+                hipLaunchKernelGGL((k_mixed_residual<decltype(NC)::value, decltype(START)::value>), k.nblk, KB, 0,
+                                   c.stream, A, seg(M_ALL), (const double *)x, b, iperm, r, k.rhs32.p, p, ra, k.x32.p);
+            });
+        };
+        residual(std::true_type{});
+        finish<3>(FIN_NONE, M_ALL);
+        poll();
+        const double rr = k.h_sc[S_D0];
+        double b_norm = std::sqrt(k.h_sc[S_D2]);
+        if (b_norm == 0.0) b_norm = 1.0;
+        *res = std::sqrt(rr) / b_norm;
+        if (!(*res >= tol)) return;
+        hipLaunchKernelGGL(k_mixed_scalars, 1, 64, 0, c.stream, k.sc.p, rr, std::max(inner_tol, tol / *res), inner_tol,
+                           b_norm, tol, (double)maxit);
+        MHFEM_HIP(hipGetLastError());
+        auto replace = [&]() {
+            with_n(c.n, [&](auto NC) {
+                hipLaunchKernelGGL((k_mixed_flush<decltype(NC)::value>), grid_for(c.F), KB, 0, c.stream, c.F,
+                                   (const double *)k.sc.p, iperm, x, k.x32.p, (const float *)p, (const float *)r, q);
+            });
+            residual(std::false_type{});
+            finish<3>(FIN_REPLACE_MERGED, M_ALL);
+        };
+        const int every = std::max(1, c.cfg.check_every);
+        const size_t bytes = NSLOTS * sizeof(double);
+        const float *continued = nullptr;  // q once the direction continues from it
+        bool ahead = false;                // the round is queued already
+        int stalls = 0;
+        for (;;) {
+            if (grouped<float>()) {
+                if (!ahead) group_iterate<float>(c, k.group, matrix<float>(), k.sc.p, k.x32.p, r, p, ra, continued);
+                replace();
+                MHFEM_HIP(hipMemcpyAsync(k.h_sc_ahead[0], k.sc.p, bytes, hipMemcpyDeviceToHost, c.stream));
+                MHFEM_HIP(hipEventRecord(k.ev_ahead[0], c.stream));
+                group_iterate<float>(c, k.group, matrix<float>(), k.sc.p, k.x32.p, r, p, ra, q);
+                ahead = true;
+                MHFEM_HIP(hipEventSynchronize(k.ev_ahead[0]));
+                std::memcpy(k.h_sc, k.h_sc_ahead[0], bytes);
+                if (k.h_sc[S_FAIL] != 0.0) {
+                    k.group.cooldown = 8;  // on with launches, from the replaced residual
+                    group_clear_failed(c, k.sc.p, 1);
+                }
+            } else {
+                if (continued)
+                    hipLaunchKernelGGL((k_bicg_pfix<float>), sg.nact, KB, 0, c.stream, sg, (const float *)r, p,
+                                       continued);
+                bicg_drive<float>(k.rhs32.p, k.x32.p, v, [&]() { bicg_iterations<float>(k.x32.p, v, every); });
+                replace();
+                poll();
+            }
+            *total = (int)k.h_sc[S_IT];
+            if (k.h_sc[S_BROKEN] != 0.0) {
+                *fallback = true;
+                return;
+            }
+            ++*outer;
+            const double prev = *res;
+            *res = std::sqrt(k.h_sc[S_D0]) / b_norm;
+            if (!(*res >= tol) || *total >= maxit) return;
+            // FP32 iterations only refine while kappa * eps_fp32 << 1: two
+            // replacements in a row that do not halve the FP64 residual
+            // hand the rest of the solve to FP64 BiCGStab
+            stalls = *res > 0.5 * prev ? stalls + 1 : 0;
+            if (stalls >= 2) {
+                *fallback = true;
+                return;
+            }
+            if (k.h_sc[S_RESTART] != 0.0) {
+                bicg_init<float>(k.rhs32.p, k.x32.p, v, M_RESTART);
+                continued = nullptr;
+                ahead = false;
+            } else {
+                continued = q;
+            }
+        }
     }
 
     // GMRES(m), FP64, one segment
@@ -3572,10 +3815,6 @@ static void parilu_factor(Ctx &c, Krylov &k)
 static void precond_update(Ctx &c, Krylov &k)
 {
     const int n = k.n;
-    const unsigned g = grid_for(n);
-    // the diagonal is 1 by construction: the Jacobi scaling is 1 / 1
-    hipLaunchKernelGGL((k_fill_t<double>), g, KB, 0, c.stream, (long)n, k.dinv.p, 1.0);
-    MHFEM_HIP(hipGetLastError());
     const bool mixed = c.cfg.precision != MHFEM_PRECISION_FP64;
     if (k.permuted64) {
         with_n(c.n, [&](auto NC) {
@@ -3597,12 +3836,10 @@ static void precond_update(Ctx &c, Krylov &k)
                 hipLaunchKernelGGL((k_convert_permuted_diag<N, float>), grid_for(c.F), KB, 0, c.stream, c.F, k.perm.p,
                                    c.sell_val.p + c.diag_base, k.val32.p + k.diag_base32);
         });
-        hipLaunchKernelGGL((k_convert<float, double>), g, KB, 0, c.stream, (long)n, k.dinv.p, k.dinv32.p);
         MHFEM_HIP(hipGetLastError());
     } else if (mixed) {
         hipLaunchKernelGGL((k_convert<float, double>), grid_for(c.sell_size), KB, 0, c.stream, c.sell_size,
                            c.sell_val.p, k.val32.p);
-        hipLaunchKernelGGL((k_convert<float, double>), g, KB, 0, c.stream, (long)n, k.dinv.p, k.dinv32.p);
         MHFEM_HIP(hipGetLastError());
     }
     if (c.cfg.preconditioner == MHFEM_PREC_AMG) amg_update(c, *k.amg);
@@ -3928,12 +4165,6 @@ void krylov_solve(Ctx &c, const double *b, double *x, mhfem_solve_stats *st)
         // applied to the FP64 residual rounded to FP32.
         float *rhs32 = k.rhs32.p, *z = k.b32.p;
         Solve::Vecs v{k.r32.p, k.r_ast32.p, k.p32.p, k.Ap32.p, k.s32.p, k.As32.p, k.tmp32.p, k.b32.p, k.dinv32.p};
-        hipLaunchKernelGGL((k_convert<float, double>), g, KB, 0, c.stream, (long)n, b, rhs32);
-        S.prec<float>(rhs32, z, k.dinv32.p, M_ALL);
-        S.dots<float, 1>(DotArgs<float, 1>{{z}, {z}}, FIN_NONE, M_ALL);
-        S.poll();
-        double b_norm = std::sqrt(k.h_sc[S_D0]);
-        if (b_norm == 0.0) b_norm = 1.0;
         const bool reliable = c.cfg.precision == MHFEM_PRECISION_FP32_RELIABLE;
         // After a solve whose FP32 iteration stalled, the next solves of the
         // trajectory (nearby systems) go straight to FP64 for a while.
@@ -3944,12 +4175,21 @@ void krylov_solve(Ctx &c, const double *b, double *x, mhfem_solve_stats *st)
         const double inner_tol = c.cfg.inner_residue > 0 ? c.cfg.inner_residue : (reliable ? 1e-2 : 1e-4);
         int total = 0, outer = 0;
         double res = 0;
-        for (; reliable && !skip_fp32;) {
-            // One FP32 recurrence with reliable updates (Sleijpen & van der
-            // Vorst 1996): each time its residual has dropped by inner_tol,
-            // the FP32 correction goes into the FP64 solution, the FP64
-            // residual replaces the recursive one and the recurrence goes on
-            // with its search direction and shadow residual.
+        const bool fused = reliable && !skip_fp32 && S.plain_prec();
+        double b_norm = 1.0;
+        if (fused) {
+            S.reliable(b, x, v, tol, maxit, inner_tol, &total, &outer, &res, &fallback);
+        } else if (!skip_fp32) {
+            hipLaunchKernelGGL((k_convert<float, double>), g, KB, 0, c.stream, (long)n, b, rhs32);
+            S.prec<float>(rhs32, z, k.dinv32.p, M_ALL);
+            S.dots<float, 1>(DotArgs<float, 1>{{z}, {z}}, FIN_NONE, M_ALL);
+            S.poll();
+            b_norm = std::sqrt(k.h_sc[S_D0]);
+            if (b_norm == 0.0) b_norm = 1.0;
+        }
+        for (; reliable && !skip_fp32 && !fused;) {
+            // the same as Solve::reliable with a preconditioner applied by
+            // its own kernels
             float *r = k.r32.p;
             S.residual_mixed(x, b, rhs32);
             S.prec<float>(rhs32, z, k.dinv32.p, M_ALL);
@@ -3960,11 +4200,7 @@ void krylov_solve(Ctx &c, const double *b, double *x, mhfem_solve_stats *st)
             hipLaunchKernelGGL((k_fill_t<float>), g, KB, 0, c.stream, (long)n, k.x32.p, 0.0f);
             S.bicg_start<float>(rhs32, k.x32.p, v, std::max(inner_tol, tol / res), maxit);
             hipLaunchKernelGGL(k_set_slots, 1, 64, 0, c.stream, k.sc.p, tol * b_norm, inner_tol);
-            // each round between two replacements gets at most `round_cap`
-            // iterations, so that a recurrence that cannot reach the next
-            // replacement still reaches the stall test below
-            const int round_cap = 300;
-            hipLaunchKernelGGL(k_set_slot, 1, 64, 0, c.stream, k.sc.p, (int)S_MAXIT, (double)std::min(maxit, round_cap));
+            hipLaunchKernelGGL(k_set_slot, 1, 64, 0, c.stream, k.sc.p, (int)S_MAXIT, (double)std::min(maxit, ROUND_CAP));
             MHFEM_HIP(hipGetLastError());
             const int every = std::max(1, c.cfg.check_every);
             int stalls = 0;
@@ -3976,21 +4212,10 @@ void krylov_solve(Ctx &c, const double *b, double *x, mhfem_solve_stats *st)
                     break;
                 }
                 S.add_correction(x, k.x32.p);
-                // the merged iteration has advanced p with the recursive
-                // residual: keep p - r for the continued direction
-                const bool merged = S.merged<float>();
-                if (merged)
-                    hipLaunchKernelGGL((k_bicg_dir<float>), k.nblk, KB, 0, c.stream, S.seg(M_ALL), (const float *)k.p32.p,
-                                       (const float *)r, k.s32.p);
                 S.residual_mixed(x, b, rhs32);
                 MHFEM_HIP(hipGetLastError());
                 S.prec<float>(rhs32, r, k.dinv32.p, M_ALL);
-                // merged: D0 = (r, r) (read below), (r, r) again in partial
-                // row 1 for the next merged alpha, D2 = (r, r*)
-                if (merged)
-                    S.dots<float, 3>(DotArgs<float, 3>{{r, r, r}, {r, r, k.r_ast32.p}}, FIN_REPLACE_MERGED, M_ALL);
-                else
-                    S.dots<float, 2>(DotArgs<float, 2>{{r, r}, {r, k.r_ast32.p}}, FIN_REPLACE, M_ALL);
+                S.dots<float, 2>(DotArgs<float, 2>{{r, r}, {r, k.r_ast32.p}}, FIN_REPLACE, M_ALL);
                 S.poll();
                 outer++;
                 const double prev = res;
@@ -4005,13 +4230,9 @@ void krylov_solve(Ctx &c, const double *b, double *x, mhfem_solve_stats *st)
                     break;
                 }
                 hipLaunchKernelGGL(k_set_slot, 1, 64, 0, c.stream, k.sc.p, (int)S_MAXIT,
-                                   (double)std::min(maxit, total + round_cap));
-                if (merged)
-                    hipLaunchKernelGGL((k_bicg_pfix<float>), S.sg.nact, KB, 0, c.stream, S.sg, (const float *)r,
-                                       k.p32.p, (const float *)k.s32.p);
-                else
-                    hipLaunchKernelGGL((k_bicg_p<float>), S.sg.nact, KB, 0, c.stream, S.sg, (const float *)r, k.p32.p,
-                                       (const float *)k.Ap32.p);
+                                   (double)std::min(maxit, total + ROUND_CAP));
+                hipLaunchKernelGGL((k_bicg_p<float>), S.sg.nact, KB, 0, c.stream, S.sg, (const float *)r, k.p32.p,
+                                   (const float *)k.Ap32.p);
                 MHFEM_HIP(hipGetLastError());
             }
             break;
