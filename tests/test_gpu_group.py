@@ -107,6 +107,19 @@ def test_batch_larger_than_the_chip():
     s.close()
 
 
+def test_rows_read_from_memory():
+    """Three species on hexahedra, past the faces whose rows fit in LDS (128
+    per CU) and below those that fit on the chip at all."""
+    pr = problems.adr_hexes(s=22, n=3)
+    assert 128 * 256 < pr.num_faces < 256 * 256
+    s = capi.Solver(pr, tol=1e-12)
+    s.step(0.0, pr.dt)
+    rp, col, val, rhs = s.export_system()
+    r = rhs - np.add.reduceat(val * s.get_array("Z_iF")[col], rp[:-1])
+    assert np.linalg.norm(r) < 2e-12 * np.linalg.norm(rhs)
+    s.close()
+
+
 def test_overlapping_contexts():
     """Two contexts solve at the same time on their own streams."""
     import threading

@@ -371,6 +371,7 @@ struct GroupTask {
 struct GroupPlan {
     int total = 0;  // work-groups, 0: the system does not fit on the chip
     int threads = 0, width = 0, nslots = 0;
+    bool lds = false;  // matrix rows in LDS
     DBuf<GroupTask> task;
     DBuf<int> seg;       // int2 per segment
     DBuf<int> face, pos; // the groups' face order and its inverse

@@ -36,7 +36,7 @@
 // launch): 64 x 64 x 2 triangles, 3 steps 3.21 -> 0.55 ms; 201 x 201 x 2,
 // 2 steps 6.37 -> 1.05 ms; 21^3 x 6 tetrahedra n = 1, 2 steps 17.7 -> 1.94 ms
 // (48 -> 4.9 us per iteration); 20^3 x 6 n = 2, FP32, 6 steps 50.5 -> 10.3 ms;
-// 32 ragged 2-D instances 40.8 -> 13.2 ms.  An exchange takes 2.4 us with 200
+// 20^3 voxels n = 3, 6.77 -> 1.33 ms; 32 ragged 2-D instances 40.8 -> 13.2 ms.  An exchange takes 2.4 us with 200
 // work-groups: 0.5 us of arithmetic, 0.4 us of work-group sums, the rest from
 // the post of the slowest work-group to its sum in every other one.  Tried:
 // neighbours polled only after the sums are in (10 us per iteration where 8
@@ -64,6 +64,12 @@ constexpr int GROUP_ND = 4;   // dot products of a reduction, at most
 // partial sums a wavefront adds, per dot product: BS / 256 wavefronts for each
 // of GROUP_ND dots cover the largest group (one work-group per CU of 256)
 constexpr int group_slots(int bs) { return bs <= 256 ? 256 : 128; }
+
+// Where a lane's matrix rows stay between products: in registers; in LDS, with
+// at most LDS_FACES faces per work-group; or in memory (the L2), read in each
+// product.
+enum { HOLD_MEMORY = 0, HOLD_REGS = 1, HOLD_LDS = 2 };
+constexpr int LDS_FACES = 128;
 
 struct GroupView {
     int total;               // work-groups of the launch
@@ -171,7 +177,7 @@ struct GroupWait {
     }
 };
 
-template <typename T, int N, int W, int BS, bool HOLD>
+template <typename T, int N, int W, int BS, int HOLD>
 __global__ void __launch_bounds__(BS) k_bicg_group(SellView<T> A, GroupView g, T *__restrict__ xg, T *__restrict__ rg,
                                                    T *__restrict__ pg, const T *__restrict__ r_ast,
                                                    const T *__restrict__ qg, T *pub)
@@ -181,6 +187,8 @@ __global__ void __launch_bounds__(BS) k_bicg_group(SellView<T> A, GroupView g, T
     __shared__ double part[2][GROUP_ND][NW], tot[2][GROUP_ND][NW / GROUP_ND];
     __shared__ Pack<T, N> mine[2][BS];  // the work-group's own published values
     __shared__ Pack<T, N> own[2][BS];   // x and r* of each lane
+    // HOLD_LDS: the matrix rows, entry by entry across the lanes with a face
+    __shared__ T rows[HOLD == HOLD_LDS ? W * N * N * LDS_FACES : 1];
     const int tid = threadIdx.x, lane = tid & 63, wid = __builtin_amdgcn_readfirstlane(tid >> 6);
     if (tid == 0) {
         s_ticket = atomicAdd(g.ticket, 1);
@@ -201,7 +209,7 @@ __global__ void __launch_bounds__(BS) k_bicg_group(SellView<T> A, GroupView g, T
 
     // ---- the face's matrix rows and its state; neighbours' p and r
     int col[W];  // the neighbour's row in the published vector, or -1 - its lane when this work-group has it
-    Pack<T, N * N> val[HOLD ? W : 1];
+    Pack<T, N * N> val[HOLD == HOLD_REGS ? W : 1];
     Pack<T, (N > 1 ? N * (N - 1) : 1)> dg;
     Pack<T, N> p, r, pn[W], rn[W];
     int w = 0;
@@ -231,14 +239,19 @@ __global__ void __launch_bounds__(BS) k_bicg_group(SellView<T> A, GroupView g, T
 #pragma unroll
     for (int k = 0; k < W; k++) {
         col[k] = k < w ? A.col[base + (int64_t)k * 64] : f;
-        if constexpr (HOLD) {
+        if constexpr (HOLD == HOLD_REGS) {
 #pragma unroll
             for (int i = 0; i < N * N; i++) val[k].v[i] = T(0);
         }
 #pragma unroll
         for (int i = 0; i < N; i++) pn[k].v[i] = rn[k].v[i] = T(0);
         if (k < w) {
-            if constexpr (HOLD) val[k] = ld<T, N * N>(A.val + (base + (int64_t)k * 64) * (N * N));
+            if constexpr (HOLD == HOLD_REGS) val[k] = ld<T, N * N>(A.val + (base + (int64_t)k * 64) * (N * N));
+            if constexpr (HOLD == HOLD_LDS) {
+                const Pack<T, N * N> row = ld<T, N * N>(A.val + (base + (int64_t)k * 64) * (N * N));
+#pragma unroll
+                for (int i = 0; i < N * N; i++) rows[(k * N * N + i) * LDS_FACES + tid] = row.v[i];
+            }
             rn[k] = ld<T, N>(rg + (int64_t)col[k] * N);
             pn[k] = direction(col[k], rn[k]);
         }
@@ -282,14 +295,21 @@ __global__ void __launch_bounds__(BS) k_bicg_group(SellView<T> A, GroupView g, T
         }
 #pragma unroll
         for (int k = 0; k < W; k++) {
-            if constexpr (!HOLD) {
+            constexpr int R = HOLD == HOLD_REGS ? 1 : 0;
+            if constexpr (HOLD == HOLD_MEMORY) {
                 if (k < w) val[0] = ld<T, N * N>(A.val + (base + (int64_t)k * 64) * (N * N));
             }
-            if (HOLD || k < w) {
+            if constexpr (HOLD == HOLD_LDS) {
+                if (k < w) {
+#pragma unroll
+                    for (int i = 0; i < N * N; i++) val[0].v[i] = rows[(k * N * N + i) * LDS_FACES + tid];
+                }
+            }
+            if (HOLD == HOLD_REGS || k < w) {
 #pragma unroll
                 for (int i = 0; i < N; i++)
 #pragma unroll
-                    for (int j = 0; j < N; j++) y.v[i] += val[HOLD ? k : 0].v[i * N + j] * nb[k].v[j];
+                    for (int j = 0; j < N; j++) y.v[i] += val[R * k].v[i * N + j] * nb[k].v[j];
             }
         }
         return y;
@@ -868,13 +888,22 @@ void with_shape(int n, int width, F &&f)
 }
 // Registers of a lane, about: a work-group of 1024 threads has 128, of 512
 // 256, of 256 512 (part of them accumulation registers).  Shapes past 400
-// read the matrix from memory in each product instead.
+// do not hold the matrix in registers.
 constexpr int lane_registers(int bytes, int n, int w) { return bytes / 4 * (n * (4 * w + 7) + n * n * (w + 1)) + w + 30; }
 constexpr int max_threads(int bytes, int n, int w)
 {
     return lane_registers(bytes, n, w) <= 92 ? 1024 : lane_registers(bytes, n, w) <= 240 ? 512 : 256;
 }
 constexpr bool holds(int bytes, int n, int w) { return lane_registers(bytes, n, w) <= 400; }
+// f(the way the matrix rows are held): registers where they fit, else LDS (when
+// the plan gives a work-group at most LDS_FACES faces) or memory
+template <typename T, int N, int W, typename F>
+void with_hold(bool lds, F &&f)
+{
+    if constexpr (holds(sizeof(T), N, W)) f(std::integral_constant<int, HOLD_REGS>{});
+    else if (lds) f(std::integral_constant<int, HOLD_LDS>{});
+    else f(std::integral_constant<int, HOLD_MEMORY>{});
+}
 template <typename T, typename F>
 void with_threads(int bs, int n, int w, F &&f)
 {
@@ -956,6 +985,14 @@ bool group_plan(Ctx &c, GroupPlan &gp, bool fp32, int width, bool gmres)
     // largest the registers allow (32 ragged instances, 1.5 M faces: 26 ms
     // with 512, 18 ms with 1024: fewer partial sums per face)
     const int bs = gmres || c.F <= 512 * cus ? std::min(512, cap_bs) : cap_bs;
+    // rows that do not fit in registers are held in LDS while one work-group of
+    // LDS_FACES faces per CU holds the system (20^3 voxels n = 3: 16.5 -> 9.7 us
+    // per iteration; a product took 3.5 us from the L2)
+    bool lds = false;
+    if (!gmres)
+        with_shape(c.n, width, [&](auto NC, auto WC) {
+            lds = !holds(fp32 ? 4 : 8, decltype(NC)::value, decltype(WC)::value) && c.F <= LDS_FACES * cus;
+        });
     int per_cu = 0;
     if (gmres)
         with_threads<double>(bs, c.n, width, [&](auto NC, auto WC, auto BC) {
@@ -965,15 +1002,21 @@ bool group_plan(Ctx &c, GroupPlan &gp, bool fp32, int width, bool gmres)
         });
     else if (fp32)
         with_threads<float>(bs, c.n, width, [&](auto NC, auto WC, auto BC) {
-            MHFEM_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(
-                &per_cu, (k_bicg_group<float, decltype(NC)::value, decltype(WC)::value, decltype(BC)::value, holds(4, decltype(NC)::value, decltype(WC)::value)>),
-                decltype(BC)::value, 0));
+            with_hold<float, decltype(NC)::value, decltype(WC)::value>(lds, [&](auto HC) {
+                MHFEM_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(
+                    &per_cu,
+                    (k_bicg_group<float, decltype(NC)::value, decltype(WC)::value, decltype(BC)::value, decltype(HC)::value>),
+                    decltype(BC)::value, 0));
+            });
         });
     else
         with_threads<double>(bs, c.n, width, [&](auto NC, auto WC, auto BC) {
-            MHFEM_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(
-                &per_cu, (k_bicg_group<double, decltype(NC)::value, decltype(WC)::value, decltype(BC)::value, holds(8, decltype(NC)::value, decltype(WC)::value)>),
-                decltype(BC)::value, 0));
+            with_hold<double, decltype(NC)::value, decltype(WC)::value>(lds, [&](auto HC) {
+                MHFEM_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(
+                    &per_cu,
+                    (k_bicg_group<double, decltype(NC)::value, decltype(WC)::value, decltype(BC)::value, decltype(HC)::value>),
+                    decltype(BC)::value, 0));
+            });
         });
     // (and as many as the wavefronts of a work-group sum)
     const long cap = std::min((long)per_cu * cus, gmres ? 256l : (long)group_slots(bs) * (bs / 256));
@@ -986,8 +1029,9 @@ bool group_plan(Ctx &c, GroupPlan &gp, bool fp32, int width, bool gmres)
         return c.h_seg_faces[a + 1] - c.h_seg_faces[a] > c.h_seg_faces[b + 1] - c.h_seg_faces[b];
     });
     auto split = [&](int F, int &G, int &fpw) {
-        G = std::max(1, (F + bs - 1) / bs);
-        fpw = std::min(bs, ((F + G - 1) / G + 63) / 64 * 64);
+        const int most = lds ? std::min(bs, LDS_FACES) : bs;
+        G = std::max(1, (F + most - 1) / most);
+        fpw = std::min(most, ((F + G - 1) / G + 63) / 64 * 64);
         G = std::max(1, (F + fpw - 1) / std::max(1, fpw));
     };
     for (int s = 0; s < nseg; s++) {
@@ -1010,6 +1054,7 @@ bool group_plan(Ctx &c, GroupPlan &gp, bool fp32, int width, bool gmres)
             tasks.push_back(GroupTask{s, q, f0 + q * fpw, std::min(f0 + F, f0 + (q + 1) * fpw)});
     }
     gp.threads = bs;
+    gp.lds = lds;
     gp.width = width;
     gp.total = (int)tasks.size();
     gp.nslots = (int)slot;
@@ -1041,8 +1086,10 @@ void group_iterate(Ctx &c, GroupPlan &gp, const SellView<T> &A, double *sc, T *x
                       sc, gp.wait_ticks};
     with_threads<T>(gp.threads, c.n, gp.width, [&](auto NC, auto WC, auto BC) {
         constexpr int BS = decltype(BC)::value;
-        hipLaunchKernelGGL((k_bicg_group<T, decltype(NC)::value, decltype(WC)::value, BS, holds(sizeof(T), decltype(NC)::value, decltype(WC)::value)>), gp.total, BS, 0, c.stream, A,
-                           v, x, r, p, r_ast, q, pub);
+        with_hold<T, decltype(NC)::value, decltype(WC)::value>(gp.lds, [&](auto HC) {
+            hipLaunchKernelGGL((k_bicg_group<T, decltype(NC)::value, decltype(WC)::value, BS, decltype(HC)::value>),
+                               gp.total, BS, 0, c.stream, A, v, x, r, p, r_ast, q, pub);
+        });
     });
     MHFEM_HIP(hipGetLastError());
 }
