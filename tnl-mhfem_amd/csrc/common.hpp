@@ -65,7 +65,8 @@ struct Coef {
 // and A x = x + (stored part) x.  Padding blocks have col = the face itself
 // and zero values; so do the entries of a face's block rows that are not in
 // that row's pattern (rows of one face may differ, e.g. a Dirichlet row).
-template <typename T>
+// PLANES: FP64, n = 2, the blocks' rows in planes (ld_planes).
+template <typename T, bool PLANES = false>
 struct SellView {
     int faces;
     const int64_t *slice_ptr;  // in blocks
@@ -134,6 +135,35 @@ template <typename T, int M>
 __device__ __forceinline__ void st(T *p, const Pack<T, M> &v)
 {
     *reinterpret_cast<Pack<T, M> *>(p) = v;
+}
+
+// An FP64 block of n = 2 is 32 bytes, two loads of a lane.  Blocks kept in
+// planes have row i of block q at (q / 64) * 256 + i * 128 + (q % 64) * 2, so that
+// each load of a wavefront reads one contiguous kilobyte and may stream;
+// interleaved, both loads touch every line of the slice, and streaming ones
+// fetch it twice.
+__host__ __device__ inline int64_t plane_row(int64_t q, int i) { return (q >> 6) * 256 + i * 128 + (q & 63) * 2; }
+template <typename T>
+__device__ __forceinline__ Pack<T, 4> ld_planes(const T *val, int64_t q)
+{
+    const Pack<T, 2> a = ld_stream<T, 2>(val + plane_row(q, 0)), b = ld_stream<T, 2>(val + plane_row(q, 1));
+    Pack<T, 4> r;
+    r.v[0] = a.v[0];
+    r.v[1] = a.v[1];
+    r.v[2] = b.v[0];
+    r.v[3] = b.v[1];
+    return r;
+}
+template <typename T>
+__device__ __forceinline__ void st_planes(T *val, int64_t q, const Pack<T, 4> &v)
+{
+    Pack<T, 2> a, b;
+    a.v[0] = v.v[0];
+    a.v[1] = v.v[1];
+    b.v[0] = v.v[2];
+    b.v[1] = v.v[3];
+    st<T, 2>(val + plane_row(q, 0), a);
+    st<T, 2>(val + plane_row(q, 1), b);
 }
 
 // Time function of a boundary model (mhfem_time_function), as the device

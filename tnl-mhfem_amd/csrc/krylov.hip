@@ -345,7 +345,7 @@ __global__ void k_init_scalars(double *sc, int nseg, double tol, double maxit)
 // loads, which leave the caches to the gathered x (whole time step of the
 // mixed-precision solve 36.9 ms; 37.9 ms at PF = 6, 38.7 ms at PF = 8,
 // 39.6 ms at PF = 3); FP64 with PF = 8 and ordinary loads (isolated product
-// 169 us; 183 us with streaming loads).  The FP32 product also loads the
+// 169 us; 183 us with streaming loads; 145 us streaming from planes).  The FP32 product also loads the
 // column indices of blocks PF and PF+1 up front, and those two blocks' values
 // and gathers as one second batch after the first blocks' products (the
 // empty asm keeps the compiler from hoisting them above those products):
@@ -353,8 +353,8 @@ __global__ void k_init_scalars(double *sc, int nseg, double tol, double maxit)
 // of an index and then a gather for each in turn (3 % more time steps per
 // second at n = 2 on 64^3; issuing the second batch with the first, 56-62
 // VGPRs, was 2 % slower).
-template <int N, typename T>
-__device__ __forceinline__ Pack<T, N> sell_face(const SellView<T> &A, const T *__restrict__ x, int E,
+template <int N, typename T, bool PLANES>
+__device__ __forceinline__ Pack<T, N> sell_face(const SellView<T, PLANES> &A, const T *__restrict__ x, int E,
                                                 Pack<T, N> &xe_out)
 {
     constexpr bool fp32 = sizeof(T) == 4;
@@ -373,10 +373,12 @@ __device__ __forceinline__ Pack<T, N> sell_face(const SellView<T> &A, const T *_
     xe_out = xe;
     Pack<T, N * N> b[PF];
     Pack<T, N> xf[PF];
+    static_assert(!PLANES || (!fp32 && N == 2), "planes hold FP64 blocks of n = 2");
 #pragma unroll
     for (int k = 0; k < PF; k++)
         if (k < w) {
-            if constexpr (fp32) b[k] = ld_stream<T, N * N>(A.val + (base + (int64_t)k * 64) * (N * N));
+            if constexpr (PLANES) b[k] = ld_planes<T>(A.val, base + (int64_t)k * 64);
+            else if constexpr (fp32) b[k] = ld_stream<T, N * N>(A.val + (base + (int64_t)k * 64) * (N * N));
             else b[k] = ld<T, N * N>(A.val + (base + (int64_t)k * 64) * (N * N));
             xf[k] = ld<T, N>(x + (int64_t)col[k] * N);
         }
@@ -418,7 +420,9 @@ __device__ __forceinline__ Pack<T, N> sell_face(const SellView<T> &A, const T *_
     }
     for (int k = PF + P2; k < w; k++) {
         const int64_t q = base + (int64_t)k * 64;
-        const Pack<T, N * N> bk = ld<T, N * N>(A.val + q * (N * N));
+        Pack<T, N * N> bk;
+        if constexpr (PLANES) bk = ld_planes<T>(A.val, q);
+        else bk = ld<T, N * N>(A.val + q * (N * N));
         const Pack<T, N> xk = ld<T, N>(x + (int64_t)A.col[q] * N);
 #pragma unroll
         for (int i = 0; i < N; i++)
@@ -429,12 +433,17 @@ __device__ __forceinline__ Pack<T, N> sell_face(const SellView<T> &A, const T *_
 }
 
 // the same without the face's own x values
-template <int N, typename T>
-__device__ __forceinline__ Pack<T, N> sell_face(const SellView<T> &A, const T *__restrict__ x, int E)
+template <int N, typename T, bool PLANES>
+__device__ __forceinline__ Pack<T, N> sell_face(const SellView<T, PLANES> &A, const T *__restrict__ x, int E)
 {
     Pack<T, N> xe;
     return sell_face<N>(A, x, E, xe);
 }
+
+template <typename V>
+constexpr bool is_planes = false;
+template <typename T>
+constexpr bool is_planes<SellView<T, true>> = true;
 
 // launch helper: f(std::integral_constant<int, n>) for the supported n
 template <typename F>
@@ -460,8 +469,8 @@ static void with_n(int n, F &&f)
 // for ND = 4 also (y, w), (z, w).  A work-group's row range holds whole
 // faces (build_blocks).
 // BS threads per work-group (256, or 512 for the FP32 product; sspmv()).
-template <typename T, int N, bool DIAG, int ND, int BS>
-__global__ void __launch_bounds__(BS) k_sspmv(SellView<T> A, Seg sg, int mode, const T *__restrict__ x,
+template <typename T, int N, bool DIAG, int ND, int BS, bool PLANES>
+__global__ void __launch_bounds__(BS) k_sspmv(SellView<T, PLANES> A, Seg sg, int mode, const T *__restrict__ x,
                                               const T *__restrict__ dinv, T *__restrict__ y, const T *__restrict__ z,
                                               const T *__restrict__ w)
 {
@@ -502,8 +511,8 @@ __global__ void __launch_bounds__(BS) k_sspmv(SellView<T> A, Seg sg, int mode, c
 }
 
 // y = b - A x on the selected segments
-template <typename T, int N>
-__global__ void __launch_bounds__(KB) k_sresidual(SellView<T> A, Seg sg, int mode, const T *__restrict__ x,
+template <typename T, int N, bool PLANES>
+__global__ void __launch_bounds__(KB) k_sresidual(SellView<T, PLANES> A, Seg sg, int mode, const T *__restrict__ x,
                                                   const T *__restrict__ b, T *__restrict__ y)
 {
     SEG_BLOCK_PROLOGUE(sg, mode);
@@ -559,8 +568,8 @@ __global__ void __launch_bounds__(KB) k_scopy2(Seg sg, int mode, const T *__rest
 // rows: r = b - A x, p = r* = r and the partial sums (r, r), (r, r) (row 1,
 // read with the first merged alpha) and (b, b), where separate kernels copied
 // b and r twice and reduced twice.
-template <typename T, int N>
-__global__ void __launch_bounds__(KB) k_bicg_start(SellView<T> A, Seg sg, const T *__restrict__ x,
+template <typename T, int N, bool PLANES>
+__global__ void __launch_bounds__(KB) k_bicg_start(SellView<T, PLANES> A, Seg sg, const T *__restrict__ x,
                                                    const T *__restrict__ b, T *__restrict__ r, T *__restrict__ p,
                                                    T *__restrict__ r_ast)
 {
@@ -898,7 +907,7 @@ __global__ void __launch_bounds__(KB) k_residual_mixed(SellView<double> A, const
 // within-face couplings of permuted face p are those of face perm[p].
 template <int N, typename TO>
 __global__ void __launch_bounds__(KB) k_convert_permuted(int64_t blocks, const int64_t *__restrict__ map,
-                                                         const double *__restrict__ src, TO *__restrict__ dst)
+                                                         const double *__restrict__ src, TO *__restrict__ dst, bool planes)
 {
     constexpr int NN = N * N;
     for (int64_t b = (int64_t)blockIdx.x * KB + threadIdx.x; b < blocks; b += (int64_t)gridDim.x * KB) {
@@ -911,6 +920,12 @@ __global__ void __launch_bounds__(KB) k_convert_permuted(int64_t blocks, const i
         } else {
 #pragma unroll
             for (int t = 0; t < NN; t++) o.v[t] = TO(0);
+        }
+        if constexpr (sizeof(TO) == 8 && N == 2) {
+            if (planes) {
+                st_planes<TO>(dst, b, o);
+                continue;
+            }
         }
         st<TO, NN>(dst + b * NN, o);
     }
@@ -1758,6 +1773,7 @@ struct Krylov {
     // the same order for the FP64 iteration: permuted FP64 matrix copy, the
     // right-hand side and iterate of the solve in that order
     bool permuted64 = false;
+    bool planes64 = false;  // its blocks in planes (ld_planes)
     DBuf<double> val64p, bp, xp;
     DBuf<int> perm, iperm, slice_width32, col32;
     DBuf<int64_t> slice_ptr32, map32;
@@ -2463,6 +2479,13 @@ Krylov *krylov_create(Ctx &c)
         build_fp32_order(c, *k);
         k->permuted = false;
         k->permuted64 = true;
+        // Planes and streaming loads where the matrix and the vectors outgrow
+        // the 256 MB last-level cache; below, ordinary loads keep it there.
+        // us per iteration, interleaved and ordinary / planes and streaming:
+        // 40^3 (143 MiB) 109 / 121, 44^3 (189 MiB) 167 / 152, 48^3 223 / 194,
+        // 56^3 377 / 318; the isolated product at 64^3 169 / 145 (4.95 and 5.77
+        // TB/s; interleaved and streaming 183).
+        k->planes64 = c.n == 2 && (int64_t)k->blocks32 * c.n * c.n * (int64_t)sizeof(double) > ((int64_t)160 << 20);
         k->val64p.alloc(k->diag_base32 + (int64_t)c.F * c.n * (c.n - 1));
         k->bp.alloc(n);
         k->xp.alloc(n);
@@ -2609,11 +2632,23 @@ struct Solve {
                               : SellView<T>{c.F, c.slice_ptr.p, c.slice_width.p, c.sell_col.p, k.val32.p, c.diag_base};
     }
 
+    // f(n, view) for the matrix of the iteration in precision T; the permuted
+    // FP64 copy may hold its blocks in planes
+    template <typename T, typename F>
+    void with_matrix(F &&f)
+    {
+        const SellView<T> A = matrix<T>();
+        if constexpr (sizeof(T) == 8)
+            if (perm64 && k.planes64)
+                return f(std::integral_constant<int, 2>{},
+                         SellView<T, true>{A.faces, A.slice_ptr, A.slice_width, A.col, A.val, A.diag_base});
+        with_n(c.n, [&](auto NC) { f(NC, A); });
+    }
+
     // launches of the matrix kernels, dispatched on the number of equations
     template <typename T, bool DIAG, int ND>
     void sspmv(const T *x, const T *dinv, T *y, const T *z, int mode, const T *w = nullptr)
     {
-        SellView<T> A = matrix<T>();
         const bool timed = kernel_timing_begin(c);
         // Threads per work-group, measured at n = 2 on the 64^3 Kuhn mesh:
         // the FP32 product runs best with 512 (one face per thread at 1024
@@ -2621,10 +2656,10 @@ struct Solve {
         // rows and 91-98 us with 1024 threads at 2048 rows); the FP64 product
         // with 256 (186 us at 512 rows; 213 us with 1024 threads at 2048).
         const int fpb = k.rows_per_block / c.n;
-        with_n(c.n, [&](auto NC) {
+        with_matrix<T>([&](auto NC, auto A) {
             auto go = [&](auto BSC) {
                 constexpr int BS = decltype(BSC)::value;
-                hipLaunchKernelGGL((k_sspmv<T, decltype(NC)::value, DIAG, ND, BS>), seg(mode).nact, BS, 0, c.stream,
+                hipLaunchKernelGGL((k_sspmv<T, decltype(NC)::value, DIAG, ND, BS, is_planes<decltype(A)>>), seg(mode).nact, BS, 0, c.stream,
                                    A, seg(mode), mode, x, dinv, y, z, w);
             };
             if (sizeof(T) == 4 && fpb >= 512) go(std::integral_constant<int, 512>{});
@@ -2636,9 +2671,8 @@ struct Solve {
     template <typename T>
     void sresidual(const T *x, const T *b, T *y, int mode)
     {
-        SellView<T> A = matrix<T>();
-        with_n(c.n, [&](auto NC) {
-            hipLaunchKernelGGL((k_sresidual<T, decltype(NC)::value>), seg(mode).nact, KB, 0, c.stream, A, seg(mode), mode, x, b, y);
+        with_matrix<T>([&](auto NC, auto A) {
+            hipLaunchKernelGGL((k_sresidual<T, decltype(NC)::value, is_planes<decltype(A)>>), seg(mode).nact, KB, 0, c.stream, A, seg(mode), mode, x, b, y);
         });
         MHFEM_HIP(hipGetLastError());
     }
@@ -2889,9 +2923,8 @@ struct Solve {
     {
         set_scalars(tol, maxit);
         if (plain_prec()) {
-            SellView<T> A = matrix<T>();
-            with_n(c.n, [&](auto NC) {
-                hipLaunchKernelGGL((k_bicg_start<T, decltype(NC)::value>), k.nblk, KB, 0, c.stream, A, seg(M_ALL),
+            with_matrix<T>([&](auto NC, auto A) {
+                hipLaunchKernelGGL((k_bicg_start<T, decltype(NC)::value, is_planes<decltype(A)>>), k.nblk, KB, 0, c.stream, A, seg(M_ALL),
                                    (const T *)x, b, (T *)v.r, (T *)v.p, (T *)v.r_ast);
             });
             finish<3>(FIN_START, M_ALL);
@@ -3820,7 +3853,7 @@ static void precond_update(Ctx &c, Krylov &k)
         with_n(c.n, [&](auto NC) {
             constexpr int N = decltype(NC)::value;
             hipLaunchKernelGGL((k_convert_permuted<N, double>), grid_for(k.blocks32), KB, 0, c.stream, k.blocks32,
-                               k.map32.p, c.sell_val.p, k.val64p.p);
+                               k.map32.p, c.sell_val.p, k.val64p.p, k.planes64);
             if constexpr (N > 1)
                 hipLaunchKernelGGL((k_convert_permuted_diag<N, double>), grid_for(c.F), KB, 0, c.stream, c.F,
                                    k.perm.p, c.sell_val.p + c.diag_base, k.val64p.p + k.diag_base32);
@@ -3831,7 +3864,7 @@ static void precond_update(Ctx &c, Krylov &k)
         with_n(c.n, [&](auto NC) {
             constexpr int N = decltype(NC)::value;
             hipLaunchKernelGGL((k_convert_permuted<N, float>), grid_for(k.blocks32), KB, 0, c.stream, k.blocks32,
-                               k.map32.p, c.sell_val.p, k.val32.p);
+                               k.map32.p, c.sell_val.p, k.val32.p, false);
             if constexpr (N > 1)
                 hipLaunchKernelGGL((k_convert_permuted_diag<N, float>), grid_for(c.F), KB, 0, c.stream, c.F, k.perm.p,
                                    c.sell_val.p + c.diag_base, k.val32.p + k.diag_base32);
