@@ -3,12 +3,11 @@ its work-groups (512 faces; 256 for three species or hexahedra), remainders,
 the smallest systems, both precisions, both face orders, batches, and the
 launched iteration that takes over when a wait in the kernel gives up.  Solved
 to 1e-13, so the oracle's solution is met to 1e-10 (the parity bar)."""
-import ctypes as C
-
 import numpy as np
 import pytest
 
 from mhfem_amd import capi, problems
+import _group
 import pyoracle
 
 pytestmark = pytest.mark.gpu
@@ -61,6 +60,7 @@ def test_one_launch_matches_oracle(case, precision, groups):
     pr = CASES[case]()
     s = capi.Solver(pr, preconditioner="diagonal", tol=1e-13, precision=precision, inner_tol=0.03, face_groups=groups)
     _steps(pr, s, pyoracle.Oracle(pr))
+    assert _group.iterated_in_one_launch(s), _group.info(s)
     s.close()
 
 
@@ -73,6 +73,7 @@ def test_gmres_cycles_match_oracle(case, restart):
     pr = CASES[case]()
     s = capi.Solver(pr, solver="gmres", preconditioner="diagonal", tol=1e-13, gmres_restart=restart)
     _steps(pr, s, pyoracle.Oracle(pr))
+    assert _group.iterated_in_one_launch(s), _group.info(s)
     s.close()
 
 
@@ -83,10 +84,11 @@ def test_a_wait_that_gives_up_hands_over(solver, precision):
     pr = problems.adr_3d(s=6, n=2, preconditioner="diagonal")
     print(f"\n[group] handed over, {solver} {precision}", flush=True)
     s = capi.Solver(pr, solver=solver, preconditioner="diagonal", tol=1e-13, precision=precision, inner_tol=0.03)
-    fn = capi.lib().mhfem_internal_group_wait
-    fn.argtypes = [C.c_void_p, C.c_ulonglong]
-    assert fn(s.ctx, 0) == 0
+    _group.wait_bound(s, 0)
     _steps(pr, s, pyoracle.Oracle(pr), steps=3)
+    i = _group.info(s)
+    # the first step's solve set eight, two more solves counted them down
+    assert (i["launches"] >= 1, i["gave_up"], i["cooldown"]) == (True, 1, 6), i
     s.close()
 
 
@@ -104,6 +106,7 @@ def test_batch_larger_than_the_chip():
     for k in range(len(members)):
         a, b = fo[k], fo[k + 1]
         assert np.linalg.norm(r[a:b]) < 2e-12 * np.linalg.norm(rhs[a:b]), k
+    assert _group.iterated_in_one_launch(s) and _group.info(s)["total"] > 256, _group.info(s)
     s.close()
 
 
@@ -117,6 +120,7 @@ def test_rows_read_from_memory():
     rp, col, val, rhs = s.export_system()
     r = rhs - np.add.reduceat(val * s.get_array("Z_iF")[col], rp[:-1])
     assert np.linalg.norm(r) < 2e-12 * np.linalg.norm(rhs)
+    assert _group.iterated_in_one_launch(s) and _group.info(s)["hold"] == "memory", _group.info(s)
     s.close()
 
 
@@ -147,4 +151,5 @@ def test_overlapping_contexts():
         t.join()
     assert not errors
     for s in solvers:
+        assert _group.iterated_in_one_launch(s), _group.info(s)
         s.close()

@@ -7,6 +7,7 @@ import numpy as np
 import pytest
 
 from mhfem_amd import capi, problems
+import _group
 
 pytestmark = pytest.mark.gpu
 
@@ -18,6 +19,7 @@ def test_planes_match_interleaved_blocks():
     for groups in (1, 0):
         print(f"\n[planes] groups {groups}", flush=True)
         s = capi.Solver(pr, preconditioner="diagonal", tol=1e-12, face_groups=groups)
+        assert _group.info(s)["planes"] == groups
         for k in range(2):
             assert s.step(k * pr.dt, pr.dt).converged
         z.append(s.get_array("Z_iF"))

@@ -1190,14 +1190,32 @@ int mhfem_guess_gradient(mhfem_ctx *ctx, const uint16_t *features, const float *
     });
 }
 
-// Test aid, not part of the interface: the bound of the waits of the
-// one-launch BiCGStab in 100 MHz ticks (0: every wait gives up at once and
-// the solve is finished by the launched iteration).
+// Test aids, not part of the interface.
+// The bound of the waits of the one-launch solves in 100 MHz ticks (0: every
+// wait gives up at once and the solve is finished by the launched iteration).
 extern "C" int mhfem_internal_group_wait(mhfem_ctx *ctx, unsigned long long ticks)
 {
     return guarded(ctx, [&](Ctx &c) {
         if (!c.system_ready) throw Error{MHFEM_E_STATE, "linear system not set up"};
         krylov_set_group_wait(*c.krylov, ticks);
+    });
+}
+// 1: the context iterates by launches also where one launch would do
+extern "C" int mhfem_internal_group_off(mhfem_ctx *ctx, int off)
+{
+    return guarded(ctx, [&](Ctx &c) {
+        if (!c.system_ready) throw Error{MHFEM_E_STATE, "linear system not set up"};
+        krylov_set_group_off(*c.krylov, off != 0);
+    });
+}
+// the first `count` values of krylov_group_info
+extern "C" int mhfem_internal_group_info(mhfem_ctx *ctx, long long *out, int count)
+{
+    return guarded(ctx, [&](Ctx &c) {
+        if (!c.system_ready) throw Error{MHFEM_E_STATE, "linear system not set up"};
+        long long v[GROUP_INFO];
+        krylov_group_info(c, *c.krylov, v);
+        for (int q = 0; q < std::min(count, (int)GROUP_INFO); q++) out[q] = v[q];
     });
 }
 

@@ -402,6 +402,7 @@ struct GroupPlan {
     int total = 0;  // work-groups, 0: the system does not fit on the chip
     int threads = 0, width = 0, nslots = 0;
     bool lds = false;  // matrix rows in LDS
+    int hold = 0;      // where the rows are held (group.hip)
     DBuf<GroupTask> task;
     DBuf<int> seg;       // int2 per segment
     DBuf<int> face, pos; // the groups' face order and its inverse
@@ -409,6 +410,11 @@ struct GroupPlan {
     DBuf<int> counters;  // ticket, beat
     DBuf<char> pub;
     int cooldown = 0;    // solves left that iterate by launches after a wait gave up
+    bool off = false;    // iterate by launches (mhfem_internal_group_off)
+    long launches = 0, gave_up = 0;  // solves, rounds or cycles in one launch; those handed over
+    // the matrix of the last launch (arrays of the context)
+    const int64_t *slice_ptr = nullptr;
+    const int *slice_width = nullptr, *col = nullptr;
     unsigned long long wait_ticks = 500000;  // 5 ms of the 100 MHz counter without any iteration in the launch
 };
 bool group_plan(Ctx &c, GroupPlan &gp, bool fp32, int width, bool gmres);
@@ -421,6 +427,15 @@ template <typename T>
 void group_iterate(Ctx &c, GroupPlan &gp, const SellView<T> &A, double *sc, T *x, T *r, T *p, const T *r_ast, const T *q);
 void group_clear_failed(Ctx &c, double *sc, int nseg);
 void krylov_set_group_wait(Krylov &k, unsigned long long ticks);
+void krylov_set_group_off(Krylov &k, bool off);
+// plan and use of the one-launch solves: [0] work-groups (0: not planned),
+// [1] threads, [2] rows held (0 memory, 1 registers, 2 LDS), [3] launches,
+// [4] of them handed over, [5] solves left by launches, [6] FP64 copy in
+// planes; of the last launch: [7] iterations, over all segments, [8] neighbours
+// its faces read, [9] those of them that are in other work-groups
+constexpr int GROUP_INFO = 10;
+void group_last(Ctx &c, GroupPlan &gp, long long *iterations, long long *neighbours, long long *remote);
+void krylov_group_info(Ctx &c, Krylov &k, long long *out);
 
 // krylov.hip
 Krylov *krylov_create(Ctx &c);

@@ -1055,6 +1055,10 @@ bool group_plan(Ctx &c, GroupPlan &gp, bool fp32, int width, bool gmres)
     }
     gp.threads = bs;
     gp.lds = lds;
+    with_shape(c.n, width, [&](auto NC, auto WC) {
+        const bool regs = holds(gmres || !fp32 ? 8 : 4, decltype(NC)::value, decltype(WC)::value);
+        gp.hold = regs ? HOLD_REGS : lds ? HOLD_LDS : HOLD_MEMORY;
+    });
     gp.width = width;
     gp.total = (int)tasks.size();
     gp.nslots = (int)slot;
@@ -1076,6 +1080,10 @@ template <typename T>
 void group_iterate(Ctx &c, GroupPlan &gp, const SellView<T> &A, double *sc, T *x, T *r, T *p, const T *r_ast,
                    const T *q)
 {
+    gp.launches++;
+    gp.slice_ptr = A.slice_ptr;
+    gp.slice_width = A.slice_width;
+    gp.col = A.col;
     const int64_t pubn = (int64_t)GROUP_ROT * c.rows;
     T *pub = reinterpret_cast<T *>(gp.pub.p);
     int *ticket = gp.counters.p;
@@ -1103,6 +1111,10 @@ int group_gmres_restart() { return GMRES_M; }
 void group_gmres_cycle(Ctx &c, GroupPlan &gp, const SellView<double> &A, double *sc, const double *r, double *x,
                        double *V, int m, double beta, double bnorm, double tol, int it, int maxit)
 {
+    gp.launches++;
+    gp.slice_ptr = A.slice_ptr;
+    gp.slice_width = A.slice_width;
+    gp.col = A.col;
     const int64_t pubn = (int64_t)GROUP_ROT * c.rows;
     double *pub = reinterpret_cast<double *>(gp.pub.p);
     int *ticket = gp.counters.p;
@@ -1117,6 +1129,39 @@ void group_gmres_cycle(Ctx &c, GroupPlan &gp, const SellView<double> &A, double 
         hipLaunchKernelGGL((k_gmres_group<N, W, BS, holds(8, N, W)>), gp.total, BS, 0, c.stream, A, v, a);
     });
     MHFEM_HIP(hipGetLastError());
+}
+
+void group_last(Ctx &c, GroupPlan &gp, long long *iterations, long long *neighbours, long long *remote)
+{
+    *iterations = *neighbours = *remote = 0;
+    if (!gp.launches) return;
+    MHFEM_HIP(hipStreamSynchronize(c.stream));
+    const int slices = (c.F + 63) / 64;
+    std::vector<int64_t> ptr(slices);
+    std::vector<int> width(slices), pos(c.F), col;
+    std::vector<GroupTask> task(gp.total);
+    unsigned beat = 0;
+    auto get = [](auto *dst, const void *src, size_t count) {
+        MHFEM_HIP(hipMemcpy(dst, src, count * sizeof(*dst), hipMemcpyDeviceToHost));
+    };
+    get(&beat, gp.counters.p + 1, 1);
+    get(ptr.data(), gp.slice_ptr, ptr.size());
+    get(width.data(), gp.slice_width, width.size());
+    get(pos.data(), gp.pos.p, pos.size());
+    get(task.data(), gp.task.p, task.size());
+    col.resize((size_t)ptr[slices - 1] + 64 * (size_t)width[slices - 1]);
+    get(col.data(), gp.col, col.size());
+    std::vector<int> group(c.F, -1);  // by position
+    for (size_t q = 0; q < task.size(); q++)
+        for (int at = task[q].p0; at < task[q].p1; at++) group[at] = (int)q;
+    for (int f = 0; f < c.F; f++)
+        for (int k = 0; k < width[f / 64]; k++) {
+            const int to = col[(size_t)ptr[f / 64] + 64 * (size_t)k + f % 64];
+            if (to == f) continue;  // padding
+            ++*neighbours;
+            *remote += group[pos[to]] != group[pos[f]];
+        }
+    *iterations = beat;
 }
 
 void group_clear_failed(Ctx &c, double *sc, int nseg)

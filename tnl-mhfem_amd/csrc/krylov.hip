@@ -2774,8 +2774,15 @@ struct Solve {
     template <typename T>
     bool grouped() const
     {
-        return k.group.total > 0 && k.group.cooldown == 0 && c.timing_level < 2 && !separate_prec() &&
+        return k.group.total > 0 && !k.group.off && k.group.cooldown == 0 && c.timing_level < 2 && !separate_prec() &&
                !jacobi_scales() && (sizeof(T) == 4) == (c.cfg.precision != MHFEM_PRECISION_FP64);
+    }
+
+    // a wait in the launch gave up: this solve and the next go on with launches
+    void hand_over()
+    {
+        k.group.cooldown = 8;
+        k.group.gave_up++;
     }
 
     // The assembled MHFEM rows are scaled so that every diagonal entry is
@@ -3002,7 +3009,7 @@ struct Solve {
                 bool failed = false;
                 for (int s = 0; s < k.nseg; s++) failed |= seg_sc(s)[S_FAIL] != 0.0;
                 if (failed) {
-                    k.group.cooldown = 8;
+                    hand_over();
                     group_clear_failed(c, k.sc.p, k.nseg);
                     break;
                 }
@@ -3129,7 +3136,7 @@ struct Solve {
                 MHFEM_HIP(hipEventSynchronize(k.ev_ahead[0]));
                 std::memcpy(k.h_sc, k.h_sc_ahead[0], bytes);
                 if (k.h_sc[S_FAIL] != 0.0) {
-                    k.group.cooldown = 8;  // on with launches, from the replaced residual
+                    hand_over();  // on with launches, from the replaced residual
                     group_clear_failed(c, k.sc.p, 1);
                 }
             } else {
@@ -3287,7 +3294,7 @@ int Solve::gmres(const double *b, double *x, double tol, int maxit, int m, doubl
             presidue<double>(x, b, V, tmp, dinv, M_ALL);
             const double norm = norm2(V);
             if (k.h_sc[S_FAIL] != 0.0) {
-                k.group.cooldown = 8;  // this solve and the next go on with launches
+                hand_over();
                 hipLaunchKernelGGL(k_set_slot, 1, 64, 0, c.stream, k.sc.p, (int)S_FAIL, 0.0);
                 MHFEM_HIP(hipGetLastError());
             } else {
@@ -3938,6 +3945,14 @@ static void precond_update(Ctx &c, Krylov &k)
 Amg *krylov_amg(const Krylov &k) { return k.amg; }
 
 void krylov_set_group_wait(Krylov &k, unsigned long long ticks) { k.group.wait_ticks = ticks; }
+void krylov_set_group_off(Krylov &k, bool off) { k.group.off = off; }
+void krylov_group_info(Ctx &c, Krylov &k, long long *out)
+{
+    GroupPlan &gp = k.group;
+    const long long v[] = {gp.total, gp.threads, gp.hold, gp.launches, gp.gave_up, gp.cooldown, k.planes64};
+    std::copy(v, v + 7, out);
+    group_last(c, gp, out + 7, out + 8, out + 9);
+}
 
 bool krylov_isai_info(const Krylov &k, long *nnz_lower, long *nnz_upper, int *rebuilds)
 {
