@@ -110,6 +110,27 @@ def test_batch_larger_than_the_chip():
     s.close()
 
 
+def test_batch_of_large_instances():
+    """Instances of 130 to 163 shares, ten of them: while one iterates the
+    work-groups left hold a part of the next, whose other shares must be taken
+    once they are free, on every XCD.  No wait gives up."""
+    sides = [3, 230, 230, 230, 230, 220, 215, 230, 210, 230, 235]
+    members = [problems.ensemble_member(sd, 40 + k) for k, sd in enumerate(sides)]
+    batch = problems.concatenate(members)
+    s = capi.Solver(batch, tol=1e-12)
+    co, fo = s.batch_info()
+    for k in range(2):
+        print(f"\n[group] large instances, step {k}", flush=True)
+        s.step(k * batch.dt, batch.dt)
+        assert _group.iterated_in_one_launch(s), _group.info(s)
+    rp, col, val, rhs = s.export_system()
+    r = rhs - np.add.reduceat(val * s.get_array("Z_iF")[col], rp[:-1])
+    for k in range(len(members)):
+        a, b = fo[k], fo[k + 1]
+        assert np.linalg.norm(r[a:b]) < 2e-12 * np.linalg.norm(rhs[a:b]), k
+    s.close()
+
+
 def test_rows_read_from_memory():
     """Three species on hexahedra, past the faces whose rows fit in LDS (128
     per CU) and below those that fit on the chip at all."""

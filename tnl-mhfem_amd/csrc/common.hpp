@@ -399,9 +399,11 @@ struct GroupTask {
     int seg, rank, p0, p1;
 };
 struct GroupPlan {
-    int total = 0;  // work-groups, 0: the system does not fit on the chip
+    int total = 0;  // shares, 0: the system does not fit on the chip
+    int resident = 0;  // work-groups that fit at once
     int threads = 0, width = 0, nslots = 0;
     bool lds = false;  // matrix rows in LDS
+    bool batch = false;
     int hold = 0;      // where the rows are held (group.hip)
     DBuf<GroupTask> task;
     DBuf<int> seg;       // int2 per segment
@@ -428,7 +430,7 @@ void group_iterate(Ctx &c, GroupPlan &gp, const SellView<T> &A, double *sc, T *x
 void group_clear_failed(Ctx &c, double *sc, int nseg);
 void krylov_set_group_wait(Krylov &k, unsigned long long ticks);
 void krylov_set_group_off(Krylov &k, bool off);
-// plan and use of the one-launch solves: [0] work-groups (0: not planned),
+// plan and use of the one-launch solves: [0] shares (0: not planned),
 // [1] threads, [2] rows held (0 memory, 1 registers, 2 LDS), [3] launches,
 // [4] of them handed over, [5] solves left by launches, [6] FP64 copy in
 // planes; of the last launch: [7] iterations, over all segments, [8] neighbours

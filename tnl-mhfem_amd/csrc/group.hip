@@ -23,9 +23,9 @@
 // * Faces are taken along a space-filling curve (group_order): most
 //   neighbours are in the same work-group and come through LDS.
 // * Work-groups take their share by ticket, the segments' shares in a row,
-//   largest segment first: the earliest unfinished segment always has all its
-//   work-groups resident once earlier ones have left, so a batch may have
-//   many more work-groups than fit at once.
+//   largest segment first, and the next one when theirs is done: the earliest
+//   unfinished segment has all its shares taken once earlier ones are done,
+//   so a batch may have many more shares than work-groups fit at once.
 // * Nothing else on the GPU is waited for: when another launch holds places
 //   that a segment needs and neither gets on, no iteration of this launch
 //   happens for 5 ms and the waits give up.  The segment is marked, every
@@ -72,7 +72,7 @@ enum { HOLD_MEMORY = 0, HOLD_REGS = 1, HOLD_LDS = 2 };
 constexpr int LDS_FACES = 128;
 
 struct GroupView {
-    int total;               // work-groups of the launch
+    int total;               // shares, one per ticket
     int64_t rows;
     const GroupTask *task;   // per ticket
     const int *face, *pos;   // the face at a position of the groups' order, and its inverse
@@ -177,10 +177,12 @@ struct GroupWait {
     }
 };
 
-template <typename T, int N, int W, int BS, int HOLD>
-__global__ void __launch_bounds__(BS) k_bicg_group(SellView<T> A, GroupView g, T *__restrict__ xg, T *__restrict__ rg,
-                                                   T *__restrict__ pg, const T *__restrict__ r_ast,
-                                                   const T *__restrict__ qg, T *pub)
+// One share of a segment, from the next ticket; false: no share is left, or a
+// wait gave up.
+template <typename T, int N, int W, int BS, int HOLD, bool BATCH>
+__device__ __forceinline__ bool bicg_share(const SellView<T> &A, const GroupView &g, T *__restrict__ xg,
+                                           T *__restrict__ rg, T *__restrict__ pg, const T *__restrict__ r_ast,
+                                           const T *__restrict__ qg, T *pub)
 {
     constexpr int NW = BS / 64, SLOTS = group_slots(BS);
     __shared__ int s_ticket, s_fail;
@@ -190,6 +192,7 @@ __global__ void __launch_bounds__(BS) k_bicg_group(SellView<T> A, GroupView g, T
     // HOLD_LDS: the matrix rows, entry by entry across the lanes with a face
     __shared__ T rows[HOLD == HOLD_LDS ? W * N * N * LDS_FACES : 1];
     const int tid = threadIdx.x, lane = tid & 63, wid = __builtin_amdgcn_readfirstlane(tid >> 6);
+    if constexpr (BATCH) __syncthreads();  // the last share's sums have been read
     if (tid == 0) {
         s_ticket = atomicAdd(g.ticket, 1);
         s_fail = 0;
@@ -197,10 +200,10 @@ __global__ void __launch_bounds__(BS) k_bicg_group(SellView<T> A, GroupView g, T
     if (tid < 2 * GROUP_ND * (NW / GROUP_ND)) (&tot[0][0][0])[tid] = 0.0;  // chunks past the group stay zero
     __syncthreads();
     const int ticket = __builtin_amdgcn_readfirstlane(s_ticket);
-    if (ticket >= g.total) return;
+    if (ticket >= g.total) return false;
     const GroupTask task = g.task[ticket];
     double *sc = g.sc + (int64_t)task.seg * NSLOTS;
-    if (halted(sc)) return;
+    if (halted(sc)) return true;
     const int G = g.seg[task.seg].y;
     double *slots = g.slots + g.seg[task.seg].x;
     const int at = task.p0 + tid;  // position in the groups' order
@@ -500,7 +503,7 @@ __global__ void __launch_bounds__(BS) k_bicg_group(SellView<T> A, GroupView g, T
             }
         if (task.rank == 0 && tid == 0) atomicAdd(g.beat, 1u);
     }
-    if (!ok) return;
+    if (!ok) return false;
     if (valid) {
         st<T, N>(xg + (int64_t)f * N, own[0][tid]);
         st<T, N>(rg + (int64_t)f * N, r);
@@ -518,6 +521,23 @@ __global__ void __launch_bounds__(BS) k_bicg_group(SellView<T> A, GroupView g, T
         sc[S_DONE] = done;
         sc[S_RESTART] = restart;
     }
+    return true;
+}
+
+// A batch: as many work-groups as fit on the chip at once, each taking share
+// after share.  (With one work-group per share, more than fit, the dispatcher
+// deals them to the 8 XCDs in turn, an XCD that has got through its eighth stays
+// idle, and what is left may not hold all of a segment's shares at once: 11
+// instances of 130-163 shares waited for each other until the waits gave up.
+// Ten instances of side 230, one step: 58 -> 42.6 ms; five of side 201: 11-33 ->
+// 9.4 ms; 32 ragged ones of 32-192, which did not: 12.1 -> 12.3 ms.)
+template <typename T, int N, int W, int BS, int HOLD, bool BATCH>
+__global__ void __launch_bounds__(BS) k_bicg_group(SellView<T> A, GroupView g, T *__restrict__ xg, T *__restrict__ rg,
+                                                   T *__restrict__ pg, const T *__restrict__ r_ast,
+                                                   const T *__restrict__ qg, T *pub)
+{
+    do {
+    } while (bicg_share<T, N, W, BS, HOLD, BATCH>(A, g, xg, rg, pg, r_ast, qg, pub) && BATCH);
 }
 
 // ---------------------------------------------------------------------------
@@ -915,6 +935,21 @@ void with_threads(int bs, int n, int w, F &&f)
     });
 }
 
+// f(the BiCGStab kernel, its threads); batches are FP64
+template <typename T, typename F>
+void with_bicg_group(int bs, int n, int width, bool lds, bool batch, F &&f)
+{
+    with_threads<T>(bs, n, width, [&](auto NC, auto WC, auto BC) {
+        constexpr int N = decltype(NC)::value, W = decltype(WC)::value, BS = decltype(BC)::value;
+        with_hold<T, N, W>(lds, [&](auto HC) {
+            constexpr int HOLD = decltype(HC)::value;
+            if constexpr (sizeof(T) == 8)
+                if (batch) return f(&k_bicg_group<T, N, W, BS, HOLD, true>, BS);
+            f(&k_bicg_group<T, N, W, BS, HOLD, false>, BS);
+        });
+    });
+}
+
 // The faces of every segment in Morton order of their positions (the lowest
 // corner of the first cell: a cell's faces stay together), so that a
 // work-group's faces are a compact piece of the mesh and few of their
@@ -993,35 +1028,21 @@ bool group_plan(Ctx &c, GroupPlan &gp, bool fp32, int width, bool gmres)
         with_shape(c.n, width, [&](auto NC, auto WC) {
             lds = !holds(fp32 ? 4 : 8, decltype(NC)::value, decltype(WC)::value) && c.F <= LDS_FACES * cus;
         });
+    const int nseg = (int)c.h_seg_faces.size() - 1;
     int per_cu = 0;
+    auto occupancy = [&](auto *kernel, int threads) {
+        MHFEM_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kernel, threads, 0));
+    };
     if (gmres)
         with_threads<double>(bs, c.n, width, [&](auto NC, auto WC, auto BC) {
             constexpr int N = decltype(NC)::value, W = decltype(WC)::value, BS = std::min(512, decltype(BC)::value);
-            MHFEM_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, (k_gmres_group<N, W, BS, holds(8, N, W)>),
-                                                                   BS, 0));
+            occupancy(k_gmres_group<N, W, BS, holds(8, N, W)>, BS);
         });
-    else if (fp32)
-        with_threads<float>(bs, c.n, width, [&](auto NC, auto WC, auto BC) {
-            with_hold<float, decltype(NC)::value, decltype(WC)::value>(lds, [&](auto HC) {
-                MHFEM_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(
-                    &per_cu,
-                    (k_bicg_group<float, decltype(NC)::value, decltype(WC)::value, decltype(BC)::value, decltype(HC)::value>),
-                    decltype(BC)::value, 0));
-            });
-        });
-    else
-        with_threads<double>(bs, c.n, width, [&](auto NC, auto WC, auto BC) {
-            with_hold<double, decltype(NC)::value, decltype(WC)::value>(lds, [&](auto HC) {
-                MHFEM_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(
-                    &per_cu,
-                    (k_bicg_group<double, decltype(NC)::value, decltype(WC)::value, decltype(BC)::value, decltype(HC)::value>),
-                    decltype(BC)::value, 0));
-            });
-        });
+    else if (fp32) with_bicg_group<float>(bs, c.n, width, lds, nseg > 1, occupancy);
+    else with_bicg_group<double>(bs, c.n, width, lds, nseg > 1, occupancy);
     // (and as many as the wavefronts of a work-group sum)
     const long cap = std::min((long)per_cu * cus, gmres ? 256l : (long)group_slots(bs) * (bs / 256));
     std::vector<GroupTask> tasks;
-    const int nseg = (int)c.h_seg_faces.size() - 1;
     std::vector<int2> segs(nseg);
     std::vector<int> order(nseg);
     for (int s = 0; s < nseg; s++) order[s] = s;
@@ -1054,6 +1075,8 @@ bool group_plan(Ctx &c, GroupPlan &gp, bool fp32, int width, bool gmres)
             tasks.push_back(GroupTask{s, q, f0 + q * fpw, std::min(f0 + F, f0 + (q + 1) * fpw)});
     }
     gp.threads = bs;
+    gp.resident = per_cu * cus;
+    gp.batch = nseg > 1;
     gp.lds = lds;
     with_shape(c.n, width, [&](auto NC, auto WC) {
         const bool regs = holds(gmres || !fp32 ? 8 : 4, decltype(NC)::value, decltype(WC)::value);
@@ -1092,12 +1115,8 @@ void group_iterate(Ctx &c, GroupPlan &gp, const SellView<T> &A, double *sc, T *x
     hipLaunchKernelGGL(k_group_prepare<T>, g, 256, 0, c.stream, pubn, pub, gp.nslots, gp.slots.p, ticket, beat);
     const GroupView v{gp.total, c.rows, gp.task.p, gp.face.p, gp.pos.p, reinterpret_cast<const int2 *>(gp.seg.p), ticket, beat, gp.slots.p,
                       sc, gp.wait_ticks};
-    with_threads<T>(gp.threads, c.n, gp.width, [&](auto NC, auto WC, auto BC) {
-        constexpr int BS = decltype(BC)::value;
-        with_hold<T, decltype(NC)::value, decltype(WC)::value>(gp.lds, [&](auto HC) {
-            hipLaunchKernelGGL((k_bicg_group<T, decltype(NC)::value, decltype(WC)::value, BS, decltype(HC)::value>),
-                               gp.total, BS, 0, c.stream, A, v, x, r, p, r_ast, q, pub);
-        });
+    with_bicg_group<T>(gp.threads, c.n, gp.width, gp.lds, gp.batch, [&](auto *kernel, int threads) {
+        hipLaunchKernelGGL(kernel, std::min(gp.total, gp.resident), threads, 0, c.stream, A, v, x, r, p, r_ast, q, pub);
     });
     MHFEM_HIP(hipGetLastError());
 }
