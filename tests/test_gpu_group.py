@@ -92,6 +92,27 @@ def test_a_wait_that_gives_up_hands_over(solver, precision):
     s.close()
 
 
+@pytest.mark.parametrize("precision", ["fp32-reliable", "fp32-refined"])
+def test_scaled_right_hand_side(precision):
+    """A right-hand side times 2^117 gives the solution times 2^117, bit for
+    bit, in as many iterations.  On edges every lane has two unused neighbour
+    slots.  Here the vectors of the first round stay below 2.2e2 (3.5e37 scaled),
+    while p carried along in an unused slot, if its neighbour's values are
+    added there, reaches 7e4 to 2.5e5 (1e40: past FP32)."""
+    pr = problems.adr_1d(s=400, n=1)
+    b = np.random.default_rng(0).standard_normal(pr.num_faces)
+    s = capi.Solver(pr, preconditioner="diagonal", tol=1e-10, precision=precision, inner_tol=1e-6)
+    s.preIterate(0.0, pr.dt)
+    s.assembleLinearSystem(0.0, pr.dt)
+    x, st = s.solve_rhs(b, np.zeros_like(b))
+    xs, sts = s.solve_rhs(b * 2.0 ** 117, np.zeros_like(b))
+    assert _group.iterated_in_one_launch(s), _group.info(s)
+    assert st.fallback_iterations == 0 and sts.fallback_iterations == 0
+    assert st.iterations == sts.iterations and st.outer_iterations == sts.outer_iterations
+    assert np.array_equal(xs, x * 2.0 ** 117)
+    s.close()
+
+
 def test_batch_larger_than_the_chip():
     """More work-groups than fit at once: segments start in turn."""
     members = [problems.ensemble_member(sd, 40 + k) for k, sd in enumerate([150, 20, 90, 150, 150, 7, 150])]

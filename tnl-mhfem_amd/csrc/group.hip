@@ -187,7 +187,7 @@ __device__ __forceinline__ bool bicg_share(const SellView<T> &A, const GroupView
     constexpr int NW = BS / 64, SLOTS = group_slots(BS);
     __shared__ int s_ticket, s_fail;
     __shared__ double part[2][GROUP_ND][NW], tot[2][GROUP_ND][NW / GROUP_ND];
-    __shared__ Pack<T, N> mine[2][BS];  // the work-group's own published values
+    __shared__ Pack<T, N> mine[2][BS + 1];  // the work-group's own published values; zeros in the last
     __shared__ Pack<T, N> own[2][BS];   // x and r* of each lane
     // HOLD_LDS: the matrix rows, entry by entry across the lanes with a face
     __shared__ T rows[HOLD == HOLD_LDS ? W * N * N * LDS_FACES : 1];
@@ -197,6 +197,9 @@ __device__ __forceinline__ bool bicg_share(const SellView<T> &A, const GroupView
         s_ticket = atomicAdd(g.ticket, 1);
         s_fail = 0;
     }
+    if (tid < 2)
+#pragma unroll
+        for (int i = 0; i < N; i++) mine[tid][BS].v[i] = T(0);
     if (tid < 2 * GROUP_ND * (NW / GROUP_ND)) (&tot[0][0][0])[tid] = 0.0;  // chunks past the group stay zero
     __syncthreads();
     const int ticket = __builtin_amdgcn_readfirstlane(s_ticket);
@@ -259,7 +262,12 @@ __device__ __forceinline__ bool bicg_share(const SellView<T> &A, const GroupView
             pn[k] = direction(col[k], rn[k]);
         }
         alone = alone && col[k] == f;
-        col[k] = k < w ? g.pos[col[k]] : task.p0;
+        // Slots past the face's width read zeros: the product multiplies
+        // them by stored zeros, and any other value kept there would follow a
+        // recurrence that the solution does not bound (one overflow, and
+        // 0 Inf = NaN).
+        col[k] = k < w ? g.pos[col[k]] : -1 - BS;
+        if (col[k] < 0) continue;
         if (col[k] < task.p0 || col[k] >= task.p1) remote |= 1u << k;
         else col[k] = -1 - (col[k] - task.p0);
     }
