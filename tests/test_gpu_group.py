@@ -3,6 +3,8 @@ its work-groups (512 faces; 256 for three species or hexahedra), remainders,
 the smallest systems, both precisions, both face orders, batches, and the
 launched iteration that takes over when a wait in the kernel gives up.  Solved
 to 1e-13, so the oracle's solution is met to 1e-10 (the parity bar)."""
+import dataclasses
+
 import numpy as np
 import pytest
 
@@ -110,6 +112,28 @@ def test_scaled_right_hand_side(precision):
     assert st.fallback_iterations == 0 and sts.fallback_iterations == 0
     assert st.iterations == sts.iterations and st.outer_iterations == sts.outer_iterations
     assert np.array_equal(xs, x * 2.0 ** 117)
+    s.close()
+
+
+def test_no_round_behind_the_end_of_a_solve():
+    """Rounds that end at nine tenths of the residual they start from do not
+    halve it: two of them hand the solve to FP64.  The round queued behind the
+    second does nothing; behind one that aims at the tolerance none is queued."""
+    pr = dataclasses.replace(problems.heat_2d(s=40), dt=10.0)
+    b = np.random.default_rng(0).standard_normal(pr.num_faces)
+    s = capi.Solver(pr, preconditioner="diagonal", tol=1e-10, precision="fp32-reliable", inner_tol=0.9)
+    s.preIterate(0.0, pr.dt)
+    s.assembleLinearSystem(0.0, pr.dt)
+    x, st = s.solve_rhs(b, np.zeros_like(b))
+    i = _group.info(s)
+    assert st.converged and st.fallback_iterations > 0
+    assert i["launches"] == st.outer_iterations + 1 and i["iterations"] == 0, (st.outer_iterations, i)
+    s.close()
+    pr = problems.heat_2d(s=40)
+    s = capi.Solver(pr, preconditioner="diagonal", tol=1e-3, precision="fp32-reliable", inner_tol=1e-3)
+    st = s.step(0.0, pr.dt)
+    i = _group.info(s)
+    assert st.outer_iterations == i["launches"] == 1 and i["iterations"] > 0, (st.outer_iterations, i)
     s.close()
 
 

@@ -148,7 +148,7 @@ __device__ __forceinline__ void memory_done()
 }
 
 // bounded waiting: gives up once nothing in the launch has iterated for
-// GROUP_WAIT_TICKS, or a work-group of the segment has given up
+// g.wait_ticks, or a work-group of the segment has given up
 struct GroupWait {
     const GroupView &g;
     double *fail;  // the segment's S_FAIL
@@ -873,12 +873,14 @@ __global__ void __launch_bounds__(BS) k_gmres_group(SellView<double> A, GroupVie
     }
 }
 
-// sentinels in the published vectors and the slots, counters at zero
+// sentinels in the published vectors and the slots, counters at zero; a
+// single segment that has stopped (sc) needs the counters only
 template <typename T>
 __global__ void __launch_bounds__(256) k_group_prepare(int64_t pubn, T *pub, int slotn, double *slots, int *ticket,
-                                                       unsigned *beat)
+                                                       unsigned *beat, const double *sc)
 {
     const int64_t stride = (int64_t)gridDim.x * 256, t = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (sc && halted(sc)) pubn = slotn = 0;
     for (int64_t i = t; i < pubn; i += stride) pub[i] = sentinel_value<T>();
     for (int64_t i = t; i < slotn; i += stride) slots[i] = sentinel_value<double>();
     if (t == 0) {
@@ -1120,7 +1122,8 @@ void group_iterate(Ctx &c, GroupPlan &gp, const SellView<T> &A, double *sc, T *x
     int *ticket = gp.counters.p;
     unsigned *beat = reinterpret_cast<unsigned *>(gp.counters.p + 1);
     const unsigned g = (unsigned)std::min<int64_t>(1024, (std::max<int64_t>(pubn, gp.nslots) + 255) / 256);
-    hipLaunchKernelGGL(k_group_prepare<T>, g, 256, 0, c.stream, pubn, pub, gp.nslots, gp.slots.p, ticket, beat);
+    hipLaunchKernelGGL(k_group_prepare<T>, g, 256, 0, c.stream, pubn, pub, gp.nslots, gp.slots.p, ticket, beat,
+                       gp.batch ? (const double *)nullptr : (const double *)sc);
     const GroupView v{gp.total, c.rows, gp.task.p, gp.face.p, gp.pos.p, reinterpret_cast<const int2 *>(gp.seg.p), ticket, beat, gp.slots.p,
                       sc, gp.wait_ticks};
     with_bicg_group<T>(gp.threads, c.n, gp.width, gp.lds, gp.batch, [&](auto *kernel, int threads) {
@@ -1147,7 +1150,8 @@ void group_gmres_cycle(Ctx &c, GroupPlan &gp, const SellView<double> &A, double 
     int *ticket = gp.counters.p;
     unsigned *beat = reinterpret_cast<unsigned *>(gp.counters.p + 1);
     const unsigned g = (unsigned)std::min<int64_t>(1024, (std::max<int64_t>(pubn, gp.nslots) + 255) / 256);
-    hipLaunchKernelGGL(k_group_prepare<double>, g, 256, 0, c.stream, pubn, pub, gp.nslots, gp.slots.p, ticket, beat);
+    hipLaunchKernelGGL(k_group_prepare<double>, g, 256, 0, c.stream, pubn, pub, gp.nslots, gp.slots.p, ticket, beat,
+                       (const double *)nullptr);
     const GroupView v{gp.total, c.rows, gp.task.p, gp.face.p, gp.pos.p, reinterpret_cast<const int2 *>(gp.seg.p),
                       ticket, beat, gp.slots.p, sc, gp.wait_ticks};
     const GmresArgs a{r, x, V, pub, m, beta, bnorm, tol, it, maxit};

@@ -202,19 +202,27 @@ __device__ void finalize(double *sc, int fin)
         // not added to the solution (k_mixed_flush) and ends the FP32 solve
         const bool again = sc[S_RESTART] != 0.0 || sc[S_FAIL] != 0.0;
         if (!isfinite(sc[S_RESID])) sc[S_BROKEN] = 1;
+        // FP32 iterations only refine while kappa * eps_fp32 << 1: two rounds
+        // in a row that do not halve the FP64 residual hand the rest of the
+        // solve to FP64 BiCGStab
+        const double res = rn / sc[S_BN0];
+        sc[S_STALLS] = res > 0.5 * sc[S_RES] ? sc[S_STALLS] + 1.0 : 0.0;
+        sc[S_RES] = res;
+        sc[S_ROUNDS] += 1;
+        sc[S_TOL] = rn > 0 ? fmax(sc[S_DELTA], sc[S_TOLABS] / rn) : 1.0;
+        sc[S_MAXIT] = fmin(sc[S_LIMIT], sc[S_IT] + ROUND_CAP);
         sc[S_RHO] = sc[S_D2];
         sc[S_BETA] = (sc[S_RHO] / sc[S_RHO_OLD]) * (sc[S_ALPHA] / sc[S_OMEGA]);
         const double fix = sc[S_BETA] / beta_old;
         sc[S_BFIX] = isfinite(fix) ? fix : 0.0;
         sc[S_BREAK] = 0;
         sc[S_BNORM] = rn;
-        sc[S_TOL] = rn > 0 ? fmax(sc[S_DELTA], sc[S_TOLABS] / rn) : 1.0;
         sc[S_RESID] = 1.0;
-        // the round ends here as the host will decide (its test on the FP64
-        // residual), so that a round queued behind it returns at once
-        sc[S_DONE] = (!(rn / sc[S_BN0] >= sc[S_TOL0]) || sc[S_IT] >= sc[S_LIMIT] || sc[S_BROKEN] != 0.0) ? 1 : 0;
+        // the solve ends here as the host will decide, so that a round queued
+        // behind it returns at once
+        sc[S_DONE] = (!(res >= sc[S_TOL0]) || sc[S_IT] >= sc[S_LIMIT] || sc[S_BROKEN] != 0.0 || sc[S_STALLS] >= 2.0)
+                         ? 1 : 0;
         sc[S_RESTART] = (rn > 0.0 && (again || !(fabs(sc[S_RHO]) >= eps2 * sc[S_RAST_SQ]))) ? 1 : 0;
-        sc[S_MAXIT] = fmin(sc[S_LIMIT], sc[S_IT] + ROUND_CAP);
         break;
     }
     default: break;
@@ -656,6 +664,7 @@ __global__ void k_mixed_scalars(double *sc, double rr, double tol_inner, double 
     sc[S_LIMIT] = limit;
     sc[S_BN0] = bn0;
     sc[S_TOL0] = tol0;
+    sc[S_RES] = sqrt(rr) / bn0;
     sc[S_DONE] = (!(1.0 >= tol_inner) || 0.0 >= limit) ? 1 : 0;
 }
 
@@ -3086,9 +3095,10 @@ struct Solve {
     // correction goes into the FP64 solution, the FP64 residual replaces the
     // recursive one and the recurrence goes on with its search direction and
     // shadow residual.  A system that iterates in one launch queues the next
-    // round before the host has read the residual of the last: the device
-    // takes the same decisions (FIN_REPLACE_MERGED), and a round queued after
-    // the end returns at once.
+    // round before the host has read the residual of the last, unless that
+    // one aims at the tolerance: the device takes the decisions
+    // (FIN_REPLACE_MERGED: tolerance, limit, breakdown, stall), and a round
+    // queued after the end returns at once.
     void reliable(const double *b, double *x, const Vecs &v, double tol, int maxit, double inner_tol, int *total,
                   int *outer, double *res, bool *fallback)
     {
@@ -3124,15 +3134,14 @@ struct Solve {
         const size_t bytes = NSLOTS * sizeof(double);
         const float *continued = nullptr;  // q once the direction continues from it
         bool ahead = false;                // the round is queued already
-        int stalls = 0;
         for (;;) {
             if (grouped<float>()) {
                 if (!ahead) group_iterate<float>(c, k.group, matrix<float>(), k.sc.p, k.x32.p, r, p, ra, continued);
                 replace();
                 MHFEM_HIP(hipMemcpyAsync(k.h_sc_ahead[0], k.sc.p, bytes, hipMemcpyDeviceToHost, c.stream));
                 MHFEM_HIP(hipEventRecord(k.ev_ahead[0], c.stream));
-                group_iterate<float>(c, k.group, matrix<float>(), k.sc.p, k.x32.p, r, p, ra, q);
-                ahead = true;
+                ahead = tol < inner_tol * *res;
+                if (ahead) group_iterate<float>(c, k.group, matrix<float>(), k.sc.p, k.x32.p, r, p, ra, q);
                 MHFEM_HIP(hipEventSynchronize(k.ev_ahead[0]));
                 std::memcpy(k.h_sc, k.h_sc_ahead[0], bytes);
                 if (k.h_sc[S_FAIL] != 0.0) {
@@ -3152,15 +3161,10 @@ struct Solve {
                 *fallback = true;
                 return;
             }
-            ++*outer;
-            const double prev = *res;
+            *outer = (int)k.h_sc[S_ROUNDS];
             *res = std::sqrt(k.h_sc[S_D0]) / b_norm;
             if (!(*res >= tol) || *total >= maxit) return;
-            // FP32 iterations only refine while kappa * eps_fp32 << 1: two
-            // replacements in a row that do not halve the FP64 residual
-            // hand the rest of the solve to FP64 BiCGStab
-            stalls = *res > 0.5 * prev ? stalls + 1 : 0;
-            if (stalls >= 2) {
+            if (k.h_sc[S_STALLS] >= 2.0) {
                 *fallback = true;
                 return;
             }
