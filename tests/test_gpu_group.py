@@ -115,6 +115,29 @@ def test_scaled_right_hand_side(precision):
     s.close()
 
 
+@pytest.mark.parametrize("case", ["tet", "edge", "tri"])
+def test_breakdown_inside_a_round(case):
+    """Values on Dirichlet faces only, from zero: (r, r*) vanishes after the
+    first iteration.  The restart belongs to its round, in one launch as by
+    launches: a solve whose only round aims at the tolerance takes one FP64
+    update, and the breakdown is no stall."""
+    pr = {"tet": lambda: problems.adr_3d(s=6, n=2, preconditioner="diagonal"), "edge": lambda: problems.adr_1d(s=60),
+          "tri": lambda: problems.adr_2d(s=18)}[case]()
+    for off in (False, True):
+        s = capi.Solver(pr, preconditioner="diagonal", tol=1e-2, precision="fp32-reliable", inner_tol=1e-2)
+        _group.launched(s, off)
+        s.preIterate(0.0, pr.dt)
+        s.assembleLinearSystem(0.0, pr.dt)
+        _, _, _, rhs = s.export_system()
+        x, st = s.solve_rhs(rhs, np.zeros_like(rhs))
+        i = _group.info(s)
+        assert st.converged and st.fallback_iterations == 0 and st.iterations > 1
+        # the round, and its second launch after the breakdown
+        assert i["gave_up"] == 0 and i["launches"] == (0 if off else 2), i
+        assert st.outer_iterations == 1, off
+        s.close()
+
+
 def test_no_round_behind_the_end_of_a_solve():
     """Rounds that end at nine tenths of the residual they start from do not
     halve it: two of them hand the solve to FP64.  The round queued behind the

@@ -197,20 +197,27 @@ __device__ void finalize(double *sc, int fin)
     case FIN_REPLACE_MERGED: {
         const double rn = sqrt(sc[S_D0]);
         const double beta_old = sc[S_BETA];
-        // a round that ended in a breakdown, or gave up (group.hip), starts
-        // afresh from the replaced residual; one whose recurrence broke was
-        // not added to the solution (k_mixed_flush) and ends the FP32 solve
+        // a recurrence that broke down in one launch, or gave up (group.hip),
+        // starts afresh from the replaced residual and its round goes on to
+        // the round's goal, as where the restart is inside the round; one that
+        // ended in non-finite numbers was not added to the solution
+        // (k_mixed_flush) and ends the FP32 solve
         const bool again = sc[S_RESTART] != 0.0 || sc[S_FAIL] != 0.0;
         if (!isfinite(sc[S_RESID])) sc[S_BROKEN] = 1;
-        // FP32 iterations only refine while kappa * eps_fp32 << 1: two rounds
-        // in a row that do not halve the FP64 residual hand the rest of the
-        // solve to FP64 BiCGStab
-        const double res = rn / sc[S_BN0];
-        sc[S_STALLS] = res > 0.5 * sc[S_RES] ? sc[S_STALLS] + 1.0 : 0.0;
-        sc[S_RES] = res;
-        sc[S_ROUNDS] += 1;
-        sc[S_TOL] = rn > 0 ? fmax(sc[S_DELTA], sc[S_TOLABS] / rn) : 1.0;
-        sc[S_MAXIT] = fmin(sc[S_LIMIT], sc[S_IT] + ROUND_CAP);
+        const double goal = sc[S_TOL] * sc[S_BNORM], res = rn / sc[S_BN0];
+        const bool same_round = again && rn > goal && sc[S_IT] < sc[S_MAXIT] && sc[S_BROKEN] == 0.0;
+        if (same_round) {
+            sc[S_TOL] = goal / rn;
+        } else {
+            // FP32 iterations only refine while kappa * eps_fp32 << 1: two
+            // rounds in a row that do not halve the FP64 residual hand the
+            // rest of the solve to FP64 BiCGStab
+            sc[S_STALLS] = res > 0.5 * sc[S_RES] ? sc[S_STALLS] + 1.0 : 0.0;
+            sc[S_RES] = res;
+            sc[S_ROUNDS] += 1;
+            sc[S_TOL] = rn > 0 ? fmax(sc[S_DELTA], sc[S_TOLABS] / rn) : 1.0;
+            sc[S_MAXIT] = fmin(sc[S_LIMIT], sc[S_IT] + ROUND_CAP);
+        }
         sc[S_RHO] = sc[S_D2];
         sc[S_BETA] = (sc[S_RHO] / sc[S_RHO_OLD]) * (sc[S_ALPHA] / sc[S_OMEGA]);
         const double fix = sc[S_BETA] / beta_old;
