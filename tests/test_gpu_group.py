@@ -66,6 +66,28 @@ def test_one_launch_matches_oracle(case, precision, groups):
     s.close()
 
 
+@pytest.mark.parametrize("precision", ["fp64", "fp32-reliable", "fp32-refined"])
+@pytest.mark.parametrize("mesh", ["tet", "tri", "hex"])
+def test_neighbours_share_work_groups(mesh, precision):
+    """Whatever the order of the matrix copy, the work-groups hold the same
+    faces, and most of a face's neighbours are in its own."""
+    pr = {"tet": lambda: problems.darcy_3d(s=12, preconditioner="diagonal"), "tri": lambda: problems.heat_2d(s=60),
+          "hex": lambda: problems.adr_hexes(s=12, n=1)}[mesh]()
+    share = []
+    for groups in (0, 1):
+        s = capi.Solver(pr, preconditioner="diagonal", tol=1e-8, precision=precision, inner_tol=1e-2,
+                        face_groups=groups)
+        assert s.step(0.0, pr.dt).converged
+        i = _group.info(s)
+        share.append(i["remote"] / i["neighbours"])
+        if groups and precision == "fp64":  # the captured step iterates on the natural order
+            s.step_graph(pr.dt, pr.dt)
+            i = _group.info(s)
+            share.append(i["remote"] / i["neighbours"])
+        s.close()
+    assert set(share) == {share[0]} and share[0] < 0.3, share
+
+
 @pytest.mark.parametrize("restart", [3, 30, 32])
 @pytest.mark.parametrize("case", sorted(CASES))
 def test_gmres_cycles_match_oracle(case, restart):

@@ -409,6 +409,7 @@ struct GroupPlan {
     DBuf<GroupTask> task;
     DBuf<int> seg;       // int2 per segment
     DBuf<int> face, pos; // the groups' face order and its inverse
+    DBuf<int> face_p, pos_p;  // the same in the numbers of the permuted matrix copy, if there is one
     DBuf<double> slots;
     DBuf<int> counters;  // ticket, beat
     DBuf<char> pub;
@@ -417,17 +418,20 @@ struct GroupPlan {
     long launches = 0, gave_up = 0;  // solves, rounds or cycles in one launch; those handed over
     // the matrix of the last launch (arrays of the context)
     const int64_t *slice_ptr = nullptr;
-    const int *slice_width = nullptr, *col = nullptr;
+    const int *slice_width = nullptr, *col = nullptr, *last_pos = nullptr;
     unsigned long long wait_ticks = 500000;  // 5 ms of the 100 MHz counter without any iteration in the launch
 };
-bool group_plan(Ctx &c, GroupPlan &gp, bool fp32, int width, bool gmres);
+// iperm: face -> its number in the permuted matrix copy (empty: there is none)
+bool group_plan(Ctx &c, GroupPlan &gp, bool fp32, int width, bool gmres, const std::vector<int> &iperm);
 // one cycle of GMRES(m) from the residual r (norm beta), m <= group_gmres_restart()
 int group_gmres_restart();
 void group_gmres_cycle(Ctx &c, GroupPlan &gp, const SellView<double> &A, double *sc, const double *r, double *x,
                        double *V, int m, double beta, double bnorm, double tol, int it, int maxit);
-// q: the direction starts as r + S_BFIX q instead of p
+// permuted: A is the permuted copy; q: the direction starts as r + S_BFIX q
+// instead of p
 template <typename T>
-void group_iterate(Ctx &c, GroupPlan &gp, const SellView<T> &A, double *sc, T *x, T *r, T *p, const T *r_ast, const T *q);
+void group_iterate(Ctx &c, GroupPlan &gp, const SellView<T> &A, bool permuted, double *sc, T *x, T *r, T *p,
+                   const T *r_ast, const T *q);
 void group_clear_failed(Ctx &c, double *sc, int nseg);
 void krylov_set_group_wait(Krylov &k, unsigned long long ticks);
 void krylov_set_group_off(Krylov &k, bool off);

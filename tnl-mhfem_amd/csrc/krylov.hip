@@ -1883,7 +1883,8 @@ struct OffsetsHash {
     }
 };
 
-static void build_fp32_order(Ctx &c, Krylov &k)
+// returns face -> its place in the order
+static std::vector<int> build_fp32_order(Ctx &c, Krylov &k)
 {
     const int F = c.F, n = c.n, nn = n * n;
     std::unordered_map<std::vector<int>, int, OffsetsHash> groups;
@@ -1958,6 +1959,7 @@ static void build_fp32_order(Ctx &c, Krylov &k)
     MHFEM_HIP(hipMemcpy(k.col32.p, col.data(), col.size() * sizeof(int), hipMemcpyHostToDevice));
     MHFEM_HIP(hipMemcpy(k.map32.p, map.data(), map.size() * sizeof(int64_t), hipMemcpyHostToDevice));
     k.permuted = true;
+    return iperm;
 }
 
 static void isai_mv(Ctx &c, const IsaiFactor &F, const double *x, double *y, const double *flag, int lanes = 0)
@@ -2486,13 +2488,14 @@ Krylov *krylov_create(Ctx &c)
         }
     }
     if (c.cfg.preconditioner == MHFEM_PREC_AMG) k->amg = amg_create();
+    std::vector<int> iperm;
     if (c.cfg.precision == MHFEM_PRECISION_FP64 && c.cfg.face_groups != 0 && k->nseg == 1 && c.unit_diagonal &&
         c.cfg.solver == MHFEM_SOLVER_BICGSTAB &&
         (c.cfg.preconditioner == MHFEM_PREC_DIAGONAL || c.cfg.preconditioner == MHFEM_PREC_NONE)) {
         // the FP64 BiCGStab iteration in the grouped face order: a permuted
         // copy of the matrix, the right-hand side and the iterate translated
         // at the start and the end of each solve
-        build_fp32_order(c, *k);
+        iperm = build_fp32_order(c, *k);
         k->permuted = false;
         k->permuted64 = true;
         // Planes and streaming loads where the matrix and the vectors outgrow
@@ -2511,7 +2514,7 @@ Krylov *krylov_create(Ctx &c)
         // the implicit unit-diagonal Jacobi (or none), the block layout
         const bool reorder = k->nseg == 1 && c.unit_diagonal && c.cfg.face_groups != 0 &&
                              (c.cfg.preconditioner == MHFEM_PREC_DIAGONAL || c.cfg.preconditioner == MHFEM_PREC_NONE);
-        if (reorder) build_fp32_order(c, *k);
+        if (reorder) iperm = build_fp32_order(c, *k);
         k->val32.alloc(k->permuted ? k->diag_base32 + (int64_t)c.F * c.n * (c.n - 1) : c.sell_size);
         for (DBuf<float> *b : {&k->dinv32, &k->b32, &k->x32, &k->r32, &k->r_ast32, &k->p32, &k->Ap32, &k->s32,
                                &k->As32, &k->tmp32, &k->rhs32})
@@ -2525,7 +2528,7 @@ Krylov *krylov_create(Ctx &c)
         (c.cfg.preconditioner == MHFEM_PREC_DIAGONAL || c.cfg.preconditioner == MHFEM_PREC_NONE)) {
         int width = 0;
         for (int E = 0; E < c.F; E++) width = std::max<int>(width, (int)(c.h_bptr[E + 1] - c.h_bptr[E]));
-        group_plan(c, k->group, c.cfg.precision != MHFEM_PRECISION_FP64, width, gmres);
+        group_plan(c, k->group, c.cfg.precision != MHFEM_PRECISION_FP64, width, gmres, iperm);
     }
     return k;
 }
@@ -2637,6 +2640,12 @@ struct Solve {
     // the FP64 BiCGStab solve runs in the grouped face order (k.permuted64)
     bool perm64 = false;
 
+    // the matrix of the iteration in precision T is a permuted copy
+    template <typename T>
+    bool permuted() const
+    {
+        return sizeof(T) == 8 ? perm64 : k.permuted;
+    }
     template <typename T>
     SellView<T> matrix()
     {
@@ -3019,7 +3028,7 @@ struct Solve {
             // segments that broke down, and takes the launched iteration
             // below when a wait in the kernel gave up
             for (;;) {
-                group_iterate<T>(c, k.group, matrix<T>(), k.sc.p, x, (T *)v.r, (T *)v.p, (const T *)v.r_ast,
+                group_iterate<T>(c, k.group, matrix<T>(), permuted<T>(), k.sc.p, x, (T *)v.r, (T *)v.p, (const T *)v.r_ast,
                                  (const T *)nullptr);
                 poll();
                 bool failed = false;
@@ -3143,12 +3152,12 @@ struct Solve {
         bool ahead = false;                // the round is queued already
         for (;;) {
             if (grouped<float>()) {
-                if (!ahead) group_iterate<float>(c, k.group, matrix<float>(), k.sc.p, k.x32.p, r, p, ra, continued);
+                if (!ahead) group_iterate<float>(c, k.group, matrix<float>(), permuted<float>(), k.sc.p, k.x32.p, r, p, ra, continued);
                 replace();
                 MHFEM_HIP(hipMemcpyAsync(k.h_sc_ahead[0], k.sc.p, bytes, hipMemcpyDeviceToHost, c.stream));
                 MHFEM_HIP(hipEventRecord(k.ev_ahead[0], c.stream));
                 ahead = tol < inner_tol * *res;
-                if (ahead) group_iterate<float>(c, k.group, matrix<float>(), k.sc.p, k.x32.p, r, p, ra, q);
+                if (ahead) group_iterate<float>(c, k.group, matrix<float>(), permuted<float>(), k.sc.p, k.x32.p, r, p, ra, q);
                 MHFEM_HIP(hipEventSynchronize(k.ev_ahead[0]));
                 std::memcpy(k.h_sc, k.h_sc_ahead[0], bytes);
                 if (k.h_sc[S_FAIL] != 0.0) {
