@@ -937,19 +937,3 @@ def test_ilut_with_p0_is_the_diagonal_and_default_beats_ilu0():
     _, _, it0, _ = pyoracle.krylov(rp, col, val, rhs, np.zeros(n), "bicgstab", "ilu0", 1e-12)
     assert conv == 1 and np.linalg.norm(x - xd) / np.linalg.norm(xd) < 1e-9
     assert it <= it0, (it, it0)
-
-
-@pytest.mark.parametrize("make", ["adr_1d", "heat_2d", "adr_quads", "darcy_3d", "adr_hexes"])
-def test_concatenated_meshes_keep_their_faces(make):
-    """The faces of a batch are its instances' faces, number by number, for
-    every cell shape (problems.concatenate)."""
-    members = [getattr(problems, make)(s=s) for s in (2, 4, 3)]
-    batch = problems.concatenate(members)
-    f0 = c0 = 0
-    for m in members:
-        assert np.array_equal(batch.cell_faces[c0:c0 + m.num_cells] - f0, m.cell_faces)
-        fc = batch.face_cells[f0:f0 + m.num_faces]
-        assert np.array_equal(np.where(fc < 0, fc, fc - c0), m.face_cells)
-        f0 += m.num_faces
-        c0 += m.num_cells
-    assert batch.num_faces == f0 and batch.num_cells == c0

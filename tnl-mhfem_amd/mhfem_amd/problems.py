@@ -457,7 +457,7 @@ def concatenate(members):
         voff += m.points.shape[0]
     points = np.concatenate(pts)
     cells = np.concatenate(cells).astype(np.int32)
-    cf, fc = meshgen.face_numbering(cells, points.shape[0], points.shape[1])
+    cf, fc = meshgen.face_numbering(cells, points.shape[0])
     lead = {"N_ijK": (n, n), "D_ijK": (n, n), "r_ijK": (n, n), "u_ijKe": (n, n, fpc), "a_ijKe": (n, n, fpc),
             "m_iK": (n,), "f_iK": (n,), "w_iKe": (n, fpc)}
     coeffs = {}
