@@ -3,6 +3,7 @@ import numpy as np
 import pytest
 
 from mhfem_amd import capi, problems
+import _group
 import pyoracle
 
 pytestmark = pytest.mark.gpu
@@ -92,6 +93,53 @@ def test_batch_narrowed_steps_equal_single_runs(check_every, rows_per_block):
             assert np.array_equal(zb[fo[j]:fo[j + 1]], z1), (k, j)
             assert np.array_equal(ka[co[j]:co[j + 1]], k1), (k, j)
             assert np.array_equal(kb[co[j]:co[j + 1]], k1), (k, j)
+
+
+LARGE = {
+    # 259,000 faces: more than work-groups of 512 threads hold at once
+    "wide": [150, 20, 90, 150, 170, 7, 60],
+    # the first does not fit on the chip: it iterates by launches, the others in one
+    "one_too_large": [300, 20, 90, 7],
+    # 1.5 M rows
+    "many": [3, 230, 230, 230, 230, 220, 215, 230, 210, 230, 235],
+}
+
+
+@pytest.mark.parametrize("off", [False, True])
+@pytest.mark.parametrize("case", ["wide", "one_too_large", "many", "tets"])
+def test_large_batch_equals_single_runs(case, off):
+    """An instance iterates bit for bit as in a context of its own, whatever
+    the batch around it: neither the share of faces of a work-group nor the
+    rows of a partial sum depends on the other instances.  In one launch and
+    by launches."""
+    if case == "tets":
+        members = [problems.adr_3d(s=v, n=2, preconditioner="diagonal") for v in (12, 4, 9, 7)]
+    else:
+        members = [problems.ensemble_member(v, 40 + k) for k, v in enumerate(LARGE[case])]
+    batch, n = problems.concatenate(members), members[0].n
+    kw = dict(preconditioner="diagonal", tol=1e-12)
+    a, b = capi.Solver(batch, **kw), capi.Solver(batch, **kw)
+    singles = [capi.Solver(m, **kw) for m in members]
+    for s in [a, b] + singles:
+        _group.launched(s, off)
+    co, fo = a.batch_info()
+    t = 0.0
+    for k in range(2):
+        print(f"\n[batch] {case} {'by launches' if off else 'in one launch'} step {k}", flush=True)
+        a.step(t, batch.dt)
+        b.step_graph(t, batch.dt)
+        its1 = np.array([s.step(t, batch.dt).iterations for s in singles])
+        t += batch.dt
+        for s in (a, b):
+            assert np.array_equal(s.batch_stats()[0], its1), k
+            z, zk = s.get_array("Z_iF").reshape(-1, n), s.get_array("Z_iK").reshape(n, -1)
+            for j, m in enumerate(singles):
+                assert np.array_equal(z[fo[j]:fo[j + 1]].ravel(), m.get_array("Z_iF")), (k, j)
+                assert np.array_equal(zk[:, co[j]:co[j + 1]].ravel(), m.get_array("Z_iK")), (k, j)
+    if not off:
+        assert _group.iterated_in_one_launch(a) and _group.iterated_in_one_launch(b), _group.info(a)
+    for s in [a, b] + singles:
+        s.close()
 
 
 @pytest.mark.parametrize("prec", ["diagonal", "ilu0"])

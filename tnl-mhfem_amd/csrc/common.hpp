@@ -395,9 +395,10 @@ void launch_zero_double(Ctx &c, double *p, size_t n);
 
 // group.hip
 // One work-group's share of a segment: the positions [p0, p1) of the groups'
-// face order, rank in the group
+// face order, in parts of `part` faces that are summed by themselves; rank:
+// the first of them among the segment's
 struct GroupTask {
-    int seg, rank, p0, p1;
+    int seg, rank, p0, p1, part;
 };
 struct GroupPlan {
     int total = 0;  // shares, 0: the system does not fit on the chip

@@ -64,6 +64,10 @@ constexpr int GROUP_ND = 4;   // dot products of a reduction, at most
 // partial sums a wavefront adds, per dot product: BS / 256 wavefronts for each
 // of GROUP_ND dots cover the largest group (one work-group per CU of 256)
 constexpr int group_slots(int bs) { return bs <= 256 ? 256 : 128; }
+// Threads of a part: a work-group of 1024 takes two parts of a segment, whose
+// sums it posts separately, so that the order of a segment's sums does not
+// depend on the threads its batch is run with.
+constexpr int part_threads(int bs) { return std::min(bs, 512); }
 
 // Where a lane's matrix rows stay between products: in registers; in LDS, with
 // at most LDS_FACES faces per work-group; or in memory (the L2), read in each
@@ -76,7 +80,7 @@ struct GroupView {
     int64_t rows;
     const GroupTask *task;   // per ticket
     const int *face, *pos;   // the face at a position of the groups' order, and its inverse
-    const int2 *seg;         // per segment: first slot (of GROUP_ROT * GROUP_ND * groups), groups
+    const int2 *seg;         // per segment: first slot (of GROUP_ROT * GROUP_ND * parts), parts
     int *ticket;             // [0]
     unsigned *beat;          // [0]: iterations of every segment of the launch
     double *slots;
@@ -177,6 +181,13 @@ struct GroupWait {
     }
 };
 
+// The arithmetic of an iteration is written out, so that every instantiation
+// (threads, where the rows are held, batch or not) gives the same bits: a
+// batch may run its instances in another one than their own contexts do.
+#pragma clang fp contract(off)
+__device__ __forceinline__ double fmadd(double a, double b, double c) { return __builtin_fma(a, b, c); }
+__device__ __forceinline__ float fmadd(float a, float b, float c) { return __builtin_fmaf(a, b, c); }
+
 // One share of a segment, from the next ticket; false: no share is left, or a
 // wait gave up.
 template <typename T, int N, int W, int BS, int HOLD, bool BATCH>
@@ -184,7 +195,7 @@ __device__ __forceinline__ bool bicg_share(const SellView<T> &A, const GroupView
                                            T *__restrict__ rg, T *__restrict__ pg, const T *__restrict__ r_ast,
                                            const T *__restrict__ qg, T *pub)
 {
-    constexpr int NW = BS / 64, SLOTS = group_slots(BS);
+    constexpr int NW = BS / 64, SLOTS = group_slots(BS), PT = part_threads(BS), NP = BS / PT;
     __shared__ int s_ticket, s_fail;
     __shared__ double part[2][GROUP_ND][NW], tot[2][GROUP_ND][NW / GROUP_ND];
     __shared__ Pack<T, N> mine[2][BS + 1];  // the work-group's own published values; zeros in the last
@@ -209,8 +220,9 @@ __device__ __forceinline__ bool bicg_share(const SellView<T> &A, const GroupView
     if (halted(sc)) return true;
     const int G = g.seg[task.seg].y;
     double *slots = g.slots + g.seg[task.seg].x;
-    const int at = task.p0 + tid;  // position in the groups' order
-    const bool valid = at < task.p1;
+    const int at = task.p0 + tid / PT * task.part + tid % PT;  // position in the groups' order
+    const bool valid = at < task.p1 && (NP == 1 || tid % PT < task.part);
+    const int parts = NP > 1 && task.p0 + task.part < task.p1 ? NP : 1;
     const int f = valid ? g.face[at] : 0;
 
     // ---- the face's matrix rows and its state; neighbours' p and r
@@ -236,7 +248,7 @@ __device__ __forceinline__ bool bicg_share(const SellView<T> &A, const GroupView
         Pack<T, N> d = ld<T, N>((qg ? qg : pg) + (int64_t)face * N);
         if (qg) {
 #pragma unroll
-            for (int i = 0; i < N; i++) d.v[i] = res.v[i] + fix * d.v[i];
+            for (int i = 0; i < N; i++) d.v[i] = fmadd(fix, d.v[i], res.v[i]);
         }
         return d;
     };
@@ -269,7 +281,10 @@ __device__ __forceinline__ bool bicg_share(const SellView<T> &A, const GroupView
         col[k] = k < w ? g.pos[col[k]] : -1 - BS;
         if (col[k] < 0) continue;
         if (col[k] < task.p0 || col[k] >= task.p1) remote |= 1u << k;
-        else col[k] = -1 - (col[k] - task.p0);
+        else {
+            const int d = col[k] - task.p0;
+            col[k] = -1 - (NP > 1 && d >= task.part ? d - task.part + PT : d);
+        }
     }
     // The pattern is symmetric but for faces without neighbours (all rows
     // Dirichlet), which their neighbours read: those faces and the ones that
@@ -302,7 +317,7 @@ __device__ __forceinline__ bool bicg_share(const SellView<T> &A, const GroupView
             for (int i = 0; i < N; i++)
 #pragma unroll
                 for (int j = 0; j < N; j++)
-                    if (j != i) y.v[i] += dg.v[i * (N - 1) + (j < i ? j : j - 1)] * own.v[j];
+                    if (j != i) y.v[i] = fmadd(dg.v[i * (N - 1) + (j < i ? j : j - 1)], own.v[j], y.v[i]);
         }
 #pragma unroll
         for (int k = 0; k < W; k++) {
@@ -320,7 +335,7 @@ __device__ __forceinline__ bool bicg_share(const SellView<T> &A, const GroupView
 #pragma unroll
                 for (int i = 0; i < N; i++)
 #pragma unroll
-                    for (int j = 0; j < N; j++) y.v[i] += val[R * k].v[i * N + j] * nb[k].v[j];
+                    for (int j = 0; j < N; j++) y.v[i] = fmadd(val[R * k].v[i * N + j], nb[k].v[j], y.v[i]);
             }
         }
         return y;
@@ -338,12 +353,16 @@ __device__ __forceinline__ bool bicg_share(const SellView<T> &A, const GroupView
         const double ws = sums_wave<ND>(acc);
         if ((lane & (64 / ND - 1)) == 0) part[par][lane / (64 / ND)][wid] = ws;
         __syncthreads();
-        if (tid < ND * GROUP_REP) {
-            double s = part[par][tid % ND][0];
+        if (tid < parts * ND * GROUP_REP) {
+            const int h = NP > 1 ? tid / (ND * GROUP_REP) : 0;
+            const double *w = part[par][tid % ND] + h * (PT / 64);
+            double s = w[0];
 #pragma unroll
-            for (int q = 1; q < NW; q++) s += part[par][tid % ND][q];
+            for (int q = 1; q < PT / 64; q++) s += w[q];
             if (is_sentinel(s)) s = __builtin_nan("");
-            coherent_store(slots + (((int64_t)(tid / ND) * GROUP_ROT + rot) * GROUP_ND + tid % ND) * G + task.rank, s);
+            coherent_store(slots + (((int64_t)(tid / ND % GROUP_REP) * GROUP_ROT + rot) * GROUP_ND + tid % ND) * G +
+                               task.rank + h,
+                           s);
         }
 #pragma unroll
         for (int k = 0; k < W; k++)
@@ -354,7 +373,7 @@ __device__ __forceinline__ bool bicg_share(const SellView<T> &A, const GroupView
         unsigned pend = remote, pd = 0;
         const int dot = wid & (ND - 1), chunk = wid / ND * SLOTS;
         const double *row =
-            slots + (((int64_t)(task.rank % GROUP_REP) * GROUP_ROT + rot) * GROUP_ND + dot) * G + chunk;
+            slots + (((int64_t)(task.rank / NP % GROUP_REP) * GROUP_ROT + rot) * GROUP_ND + dot) * G + chunk;
         double v[SLOTS / 64];
 #pragma unroll
         for (int q = 0; q < SLOTS / 64; q++) {
@@ -401,9 +420,10 @@ __device__ __forceinline__ bool bicg_share(const SellView<T> &A, const GroupView
         // previous one: its copies are cleared, for epoch e + 3
         const int old = (e + GROUP_ROT - 1) & (GROUP_ROT - 1);
         if (shared_face) unpublish<T, N>(pub + (int64_t)old * g.rows + (int64_t)at * N);
-        if (tid < GROUP_ND * GROUP_REP)
-            coherent_store(slots + (((int64_t)(tid / GROUP_ND) * GROUP_ROT + old) * GROUP_ND + tid % GROUP_ND) * G +
-                               task.rank,
+        if (tid < parts * GROUP_ND * GROUP_REP)
+            coherent_store(slots +
+                               (((int64_t)(tid / GROUP_ND % GROUP_REP) * GROUP_ROT + old) * GROUP_ND + tid % GROUP_ND) * G +
+                               task.rank + (NP > 1 ? tid / (GROUP_ND * GROUP_REP) : 0),
                            sentinel_value<double>());
         e++;
         return s_fail == 0;
@@ -426,8 +446,8 @@ __device__ __forceinline__ bool bicg_share(const SellView<T> &A, const GroupView
         double d2[2] = {0.0, 0.0};
 #pragma unroll
         for (int i = 0; i < N; i++) {
-            d2[0] += (double)Ap.v[i] * (double)ra.v[i];
-            d2[1] += (double)r.v[i] * (double)r.v[i];
+            d2[0] = fmadd((double)Ap.v[i], (double)ra.v[i], d2[0]);
+            d2[1] = fmadd((double)r.v[i], (double)r.v[i], d2[1]);
         }
         if (!valid) d2[0] = d2[1] = 0.0;
         ok = exchange(Ap, d2, std::integral_constant<int, 2>{}, an);
@@ -457,11 +477,11 @@ __device__ __forceinline__ bool bicg_share(const SellView<T> &A, const GroupView
         const T al = (T)alpha;
         Pack<T, N> s;
 #pragma unroll
-        for (int i = 0; i < N; i++) s.v[i] = r.v[i] - al * Ap.v[i];
+        for (int i = 0; i < N; i++) s.v[i] = fmadd(-al, Ap.v[i], r.v[i]);
 #pragma unroll
         for (int k = 0; k < W; k++)
 #pragma unroll
-            for (int i = 0; i < N; i++) rn[k].v[i] = rn[k].v[i] - al * an[k].v[i];
+            for (int i = 0; i < N; i++) rn[k].v[i] = fmadd(-al, an[k].v[i], rn[k].v[i]);
         // ---- As, (As, s), (As, As), (As, r*), (s, r*)
         const Pack<T, N> As = product(s, rn);
         const Pack<T, N> rb = own[1][tid];
@@ -469,10 +489,10 @@ __device__ __forceinline__ bool bicg_share(const SellView<T> &A, const GroupView
 #pragma unroll
         for (int i = 0; i < N; i++) {
             const double av = As.v[i], sv = s.v[i], rv = rb.v[i];
-            d4[0] += av * sv;
-            d4[1] += av * av;
-            d4[2] += av * rv;
-            d4[3] += sv * rv;
+            d4[0] = fmadd(av, sv, d4[0]);
+            d4[1] = fmadd(av, av, d4[1]);
+            d4[2] = fmadd(av, rv, d4[2]);
+            d4[3] = fmadd(sv, rv, d4[3]);
         }
         if (!valid) d4[0] = d4[1] = d4[2] = d4[3] = 0.0;
         ok = exchange(As, d4, std::integral_constant<int, 4>{}, a2);
@@ -481,7 +501,7 @@ __device__ __forceinline__ bool bicg_share(const SellView<T> &A, const GroupView
             const double D[4] = {total(0), total(1), total(2), total(3)};
             // beta = (rho / rho_old) (alpha / omega) with alpha / rho_old = 1 / (r*, Ap)
             const double om = uniform(D[1] > 0 ? D[0] / D[1] : 0.0), inv_om = uniform(D[1] / D[0]);
-            const double rn_ = uniform(D[3] - om * D[2]);
+            const double rn_ = uniform(fmadd(-om, D[2], D[3]));
             omega = om;
             it += 1.0;
             rho_old = rho;
@@ -497,17 +517,17 @@ __device__ __forceinline__ bool bicg_share(const SellView<T> &A, const GroupView
         Pack<T, N> x = own[0][tid];
 #pragma unroll
         for (int i = 0; i < N; i++) {
-            x.v[i] += al * p.v[i] + om * s.v[i];
-            r.v[i] = s.v[i] - om * As.v[i];
-            p.v[i] = r.v[i] + be * (p.v[i] - om * Ap.v[i]);
+            x.v[i] += fmadd(al, p.v[i], om * s.v[i]);
+            r.v[i] = fmadd(-om, As.v[i], s.v[i]);
+            p.v[i] = fmadd(be, fmadd(-om, Ap.v[i], p.v[i]), r.v[i]);
         }
         own[0][tid] = x;
 #pragma unroll
         for (int k = 0; k < W; k++)
 #pragma unroll
             for (int i = 0; i < N; i++) {
-                rn[k].v[i] = rn[k].v[i] - om * a2[k].v[i];
-                pn[k].v[i] = rn[k].v[i] + be * (pn[k].v[i] - om * an[k].v[i]);
+                rn[k].v[i] = fmadd(-om, a2[k].v[i], rn[k].v[i]);
+                pn[k].v[i] = fmadd(be, fmadd(-om, an[k].v[i], pn[k].v[i]), rn[k].v[i]);
             }
         if (task.rank == 0 && tid == 0) atomicAdd(g.beat, 1u);
     }
@@ -532,13 +552,15 @@ __device__ __forceinline__ bool bicg_share(const SellView<T> &A, const GroupView
     return true;
 }
 
+#pragma clang fp contract(fast)
+
 // A batch: as many work-groups as fit on the chip at once, each taking share
 // after share.  (With one work-group per share, more than fit, the dispatcher
 // deals them to the 8 XCDs in turn, an XCD that has got through its eighth stays
 // idle, and what is left may not hold all of a segment's shares at once: 11
 // instances of 130-163 shares waited for each other until the waits gave up.
-// Ten instances of side 230, one step: 58 -> 42.6 ms; five of side 201: 11-33 ->
-// 9.4 ms; 32 ragged ones of 32-192, which did not: 12.1 -> 12.3 ms.)
+// Ten instances of side 230, one step: 55.6-58 -> 32.9 ms; five of side 201:
+// 11-33 -> 9.8 ms; 32 ragged ones of 32-192, where no wait gave up: 12.0 -> 11.4 ms.)
 template <typename T, int N, int W, int BS, int HOLD, bool BATCH>
 __global__ void __launch_bounds__(BS) k_bicg_group(SellView<T> A, GroupView g, T *__restrict__ xg, T *__restrict__ rg,
                                                    T *__restrict__ pg, const T *__restrict__ r_ast,
@@ -945,7 +967,8 @@ void with_threads(int bs, int n, int w, F &&f)
     });
 }
 
-// f(the BiCGStab kernel, its threads); batches are FP64
+constexpr int BATCH_WIDTH = 6;
+// f(the BiCGStab kernel, its threads); batches are FP64 and on simplices
 template <typename T, typename F>
 void with_bicg_group(int bs, int n, int width, bool lds, bool batch, F &&f)
 {
@@ -953,7 +976,7 @@ void with_bicg_group(int bs, int n, int width, bool lds, bool batch, F &&f)
         constexpr int N = decltype(NC)::value, W = decltype(WC)::value, BS = decltype(BC)::value;
         with_hold<T, N, W>(lds, [&](auto HC) {
             constexpr int HOLD = decltype(HC)::value;
-            if constexpr (sizeof(T) == 8)
+            if constexpr (sizeof(T) == 8 && W <= BATCH_WIDTH)
                 if (batch) return f(&k_bicg_group<T, N, W, BS, HOLD, true>, BS);
             f(&k_bicg_group<T, N, W, BS, HOLD, false>, BS);
         });
@@ -1025,20 +1048,44 @@ bool group_plan(Ctx &c, GroupPlan &gp, bool fp32, int width, bool gmres, const s
     }();
     int cus = 0;
     MHFEM_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, c.device));
+    const int nseg = (int)c.h_seg_faces.size() - 1;
+    if (nseg > 1 && width > BATCH_WIDTH) return false;
+    bool regs = true;
+    with_shape(c.n, width, [&](auto NC, auto WC) {
+        regs = holds(gmres || !fp32 ? 8 : 4, decltype(NC)::value, decltype(WC)::value);
+    });
+    // Faces of a part, at most, by the faces of its segment alone: an instance
+    // is summed in a batch as in a context of its own.  Rows that do not fit
+    // in registers are held in LDS while one work-group of LDS_FACES faces per
+    // CU holds the segment (20^3 voxels n = 3: 16.5 -> 9.7 us per iteration; a
+    // product took 3.5 us from the L2).
+    auto most = [&](int F) {
+        return !regs && !gmres && F <= LDS_FACES * cus ? LDS_FACES : part_threads(cap_bs);
+    };
+    auto split = [&](int F, int &G, int &part) {
+        G = std::max(1, (F + most(F) - 1) / most(F));
+        part = std::min(most(F), ((F + G - 1) / G + 63) / 64 * 64);
+        G = std::max(1, (F + part - 1) / std::max(1, part));
+    };
     // 512 threads while one such work-group per CU holds every face (64 x 64
     // x 2 triangles: 0.63 ms with 512, 0.76 ms with 1024); more faces take the
-    // largest the registers allow (32 ragged instances, 1.5 M faces: 26 ms
-    // with 512, 18 ms with 1024: fewer partial sums per face)
-    const int bs = gmres || c.F <= 512 * cus ? std::min(512, cap_bs) : cap_bs;
-    // rows that do not fit in registers are held in LDS while one work-group of
-    // LDS_FACES faces per CU holds the system (20^3 voxels n = 3: 16.5 -> 9.7 us
-    // per iteration; a product took 3.5 us from the L2)
-    bool lds = false;
-    if (!gmres)
-        with_shape(c.n, width, [&](auto NC, auto WC) {
-            lds = !holds(fp32 ? 4 : 8, decltype(NC)::value, decltype(WC)::value) && c.F <= LDS_FACES * cus;
-        });
-    const int nseg = (int)c.h_seg_faces.size() - 1;
+    // largest the registers allow (32 ragged instances, 1.5 M faces: 16.7 ms
+    // with 512 and two work-groups per CU, 11.4 with 1024)
+    const int bs = gmres || c.F <= 512 * cus ? std::min(512, cap_bs) : cap_bs, np = bs / part_threads(bs);
+    // the segments whose shares fit on the chip at once are planned; the
+    // others of a batch iterate by launches afterwards
+    bool lds = !regs && !gmres;
+    const int cap = std::min(cus, 256);
+    std::vector<int> order;
+    for (int s = 0; s < nseg; s++) {
+        const int F = c.h_seg_faces[s + 1] - c.h_seg_faces[s];
+        int G, part;
+        split(F, G, part);
+        if ((G + np - 1) / np > cap) continue;
+        order.push_back(s);
+        lds = lds && F <= LDS_FACES * cus;
+    }
+    if (order.empty()) return false;
     int per_cu = 0;
     auto occupancy = [&](auto *kernel, int threads) {
         MHFEM_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kernel, threads, 0));
@@ -1050,47 +1097,30 @@ bool group_plan(Ctx &c, GroupPlan &gp, bool fp32, int width, bool gmres, const s
         });
     else if (fp32) with_bicg_group<float>(bs, c.n, width, lds, nseg > 1, occupancy);
     else with_bicg_group<double>(bs, c.n, width, lds, nseg > 1, occupancy);
-    // (and as many as the wavefronts of a work-group sum)
-    const long cap = std::min((long)per_cu * cus, gmres ? 256l : (long)group_slots(bs) * (bs / 256));
+    if (per_cu < 1) return false;
     std::vector<GroupTask> tasks;
-    std::vector<int2> segs(nseg);
-    std::vector<int> order(nseg);
-    for (int s = 0; s < nseg; s++) order[s] = s;
+    std::vector<int2> segs(nseg, int2{0, 0});
     std::stable_sort(order.begin(), order.end(), [&](int a, int b) {
         return c.h_seg_faces[a + 1] - c.h_seg_faces[a] > c.h_seg_faces[b + 1] - c.h_seg_faces[b];
     });
-    auto split = [&](int F, int &G, int &fpw) {
-        const int most = lds ? std::min(bs, LDS_FACES) : bs;
-        G = std::max(1, (F + most - 1) / most);
-        fpw = std::min(most, ((F + G - 1) / G + 63) / 64 * 64);
-        G = std::max(1, (F + fpw - 1) / std::max(1, fpw));
-    };
-    for (int s = 0; s < nseg; s++) {
-        int G, fpw;
-        split(c.h_seg_faces[s + 1] - c.h_seg_faces[s], G, fpw);
-        if (G > cap) return false;
-    }
     // positions: each segment's faces along a space-filling curve
     std::vector<int> face(c.F), pos(c.F);
     group_order(c, face);
     long slot = 0;
     for (int s : order) {
         const int f0 = c.h_seg_faces[s], F = c.h_seg_faces[s + 1] - f0;
-        int G, fpw;
-        split(F, G, fpw);
+        int G, part;
+        split(F, G, part);
         segs[s] = int2{(int)slot, G};
         slot += gmres ? (long)GROUP_ROT * GMRES_M * G : (long)GROUP_REP * GROUP_ROT * GROUP_ND * G;
-        for (int q = 0; q < G; q++)
-            tasks.push_back(GroupTask{s, q, f0 + q * fpw, std::min(f0 + F, f0 + (q + 1) * fpw)});
+        for (int q = 0; q < G; q += np)
+            tasks.push_back(GroupTask{s, q, f0 + q * part, std::min(f0 + F, f0 + (q + np) * part), part});
     }
     gp.threads = bs;
     gp.resident = per_cu * cus;
     gp.batch = nseg > 1;
     gp.lds = lds;
-    with_shape(c.n, width, [&](auto NC, auto WC) {
-        const bool regs = holds(gmres || !fp32 ? 8 : 4, decltype(NC)::value, decltype(WC)::value);
-        gp.hold = regs ? HOLD_REGS : lds ? HOLD_LDS : HOLD_MEMORY;
-    });
+    gp.hold = regs ? HOLD_REGS : lds ? HOLD_LDS : HOLD_MEMORY;
     gp.width = width;
     gp.total = (int)tasks.size();
     gp.nslots = (int)slot;

@@ -1815,8 +1815,8 @@ struct Krylov {
 
 static inline unsigned grid_for(long n) { return (unsigned)std::max<long>(1, std::min<long>((n + KB - 1) / KB, MAXG)); }
 
-// Rows per work-group when the caller names none: about 1500 work-groups, so
-// that small systems still fill the CUs (with 2048 rows 169,000 unknowns made
+// Rows per work-group when the caller names none: about 1500 work-groups per
+// segment, so that small systems still fill the CUs (with 2048 rows 169,000 unknowns made
 // 83 work-groups), within 512 and 2048 rows (more partial sums cost the
 // reductions more than smaller work-groups gain).  Measured, us per iteration
 // with 512 / 1024 / 2048 rows: 669,000 unknowns FP64 n = 2 64.3 / 64.1 / 75.9;
@@ -1831,14 +1831,17 @@ static int default_rows(int rows)
     return rpb;
 }
 
-// work-group tables for `rpb` rows per work-group, segment aligned
-static void build_blocks(Ctx &c, Krylov &k, int rpb)
+// work-group tables for `rows` rows per work-group, segment aligned; 0: each
+// segment's default, so that an instance is summed in a batch as alone
+static void build_blocks(Ctx &c, Krylov &k, int rows)
 {
-    // whole faces per work-group: the matrix kernels run one lane per face
-    rpb = std::max(c.n, rpb / c.n * c.n);
     std::vector<int> bseg, brow, sblk(1, 0);
+    k.rows_per_block = 0;
     for (int s = 0; s < k.nseg; s++) {
         const int r0 = c.h_seg_rows[s], r1 = c.h_seg_rows[s + 1];
+        // whole faces per work-group: the matrix kernels run one lane per face
+        const int rpb = std::max(c.n, (rows > 0 ? rows : default_rows(r1 - r0)) / c.n * c.n);
+        k.rows_per_block = std::max(k.rows_per_block, rpb);
         for (int r = r0; r < r1; r += rpb) {
             bseg.push_back(s);
             brow.push_back(r);
@@ -1853,7 +1856,6 @@ static void build_blocks(Ctx &c, Krylov &k, int rpb)
     // brow[b + 1] is the end of work-group b: the next work-group starts where
     // this one ends, and every segment's first work-group starts at its first row
     k.nblk = (int)bseg.size();
-    k.rows_per_block = rpb;
     k.blk_seg.alloc(k.nblk);
     k.blk_row.alloc(k.nblk + 1);
     k.seg_blk.alloc(k.nseg + 1);
@@ -2467,7 +2469,7 @@ Krylov *krylov_create(Ctx &c)
     // the diagonal is 1 by construction: the Jacobi scaling is 1 / 1
     hipLaunchKernelGGL((k_fill_t<double>), grid_for(n), KB, 0, c.stream, (long)n, k->dinv.p, 1.0);
     MHFEM_HIP(hipGetLastError());
-    build_blocks(c, *k, c.cfg.rows_per_block > 0 ? c.cfg.rows_per_block : default_rows(n));
+    build_blocks(c, *k, c.cfg.rows_per_block);
     if (c.cfg.preconditioner == MHFEM_PREC_ILUT) k->ilu.a0.alloc(c.nnz);
     // level tables: ILU(0), the ISAI factors and SOR's sweeps
     if (c.cfg.preconditioner == MHFEM_PREC_ILU0 || is_isai(c.cfg.preconditioner) || c.cfg.solver == MHFEM_SOLVER_SOR) {
@@ -3024,9 +3026,10 @@ struct Solve {
     int bicg_drive(const T *b, T *x, const Vecs &v, More &&more)
     {
         if (grouped<T>()) {
-            // every segment iterates inside one launch; the host restarts
-            // segments that broke down, and takes the launched iteration
-            // below when a wait in the kernel gave up
+            // every segment that fits iterates inside one launch; the host
+            // restarts segments that broke down, and takes the launched
+            // iteration below for segments that do not fit, or when a wait in
+            // the kernel gave up
             for (;;) {
                 group_iterate<T>(c, k.group, matrix<T>(), permuted<T>(), k.sc.p, x, (T *)v.r, (T *)v.p, (const T *)v.r_ast,
                                  (const T *)nullptr);
@@ -3039,6 +3042,7 @@ struct Solve {
                     break;
                 }
                 if (all_done()) return most_iterations();
+                if (!any_restart()) break;
                 bicg_init<T>(b, x, v, M_RESTART);
             }
         }
