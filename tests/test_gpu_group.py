@@ -104,15 +104,24 @@ def test_gmres_cycles_match_oracle(case, restart):
 @pytest.mark.parametrize("solver,precision", [("bicgstab", "fp64"), ("bicgstab", "fp32-reliable"), ("gmres", "fp64")])
 def test_a_wait_that_gives_up_hands_over(solver, precision):
     """With a bound of zero the first wait between two work-groups gives up:
-    the solve is finished by the launched iteration, and so are the next ones."""
+    the solve is finished by the launched iteration, the next one tries one
+    launch again, and after two in a row that gave up one does not.  With the
+    bound back, solves run in one launch again."""
     pr = problems.adr_3d(s=6, n=2, preconditioner="diagonal")
     print(f"\n[group] handed over, {solver} {precision}", flush=True)
     s = capi.Solver(pr, solver=solver, preconditioner="diagonal", tol=1e-13, precision=precision, inner_tol=0.03)
     _group.wait_bound(s, 0)
     _steps(pr, s, pyoracle.Oracle(pr), steps=3)
     i = _group.info(s)
-    # the first step's solve set eight, two more solves counted them down
-    assert (i["launches"] >= 1, i["gave_up"], i["cooldown"]) == (True, 1, 6), i
+    # the second solve tries one launch again, the third does not
+    assert (i["gave_up"], i["cooldown"]) == (2, 1) and i["launches"] >= 2, i
+    _group.wait_bound(s, 500000)
+    t = 3 * pr.dt
+    for k in range(2):
+        assert s.step(t, pr.dt).converged
+        t += pr.dt
+    j = _group.info(s)
+    assert j["gave_up"] == 2 and j["cooldown"] == 0 and j["launches"] > i["launches"], j
     s.close()
 
 

@@ -415,6 +415,7 @@ struct GroupPlan {
     DBuf<int> counters;  // ticket, beat
     DBuf<char> pub;
     int cooldown = 0;    // solves left that iterate by launches after a wait gave up
+    int penalty = 1;     // the next cooldown
     bool off = false;    // iterate by launches (mhfem_internal_group_off)
     long launches = 0, gave_up = 0;  // solves, rounds or cycles in one launch; those handed over
     // the matrix of the last launch (arrays of the context)

@@ -30,7 +30,8 @@
 //   that a segment needs and neither gets on, no iteration of this launch
 //   happens for 5 ms and the waits give up.  The segment is marked, every
 //   work-group leaves, and the host restarts it with the launched iteration
-//   from the iterate it has (and keeps to that for the next solves).
+//   from the iterate it has (and keeps to that for some solves where the
+//   next try gives up too).
 //
 // Measured (MI355X, whole trajectories as in perf/cases.py, launched -> one
 // launch): 64 x 64 x 2 triangles, 3 steps 3.21 -> 0.55 ms; 201 x 201 x 2,

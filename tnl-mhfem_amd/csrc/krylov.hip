@@ -2805,12 +2805,22 @@ struct Solve {
                !jacobi_scales() && (sizeof(T) == 4) == (c.cfg.precision != MHFEM_PRECISION_FP64);
     }
 
-    // a wait in the launch gave up: this solve and the next go on with launches
+    // A wait in the launch gave up: this solve goes on with launches, and so
+    // do the next ones if the last try gave up too (1, 3, 7, ... 31 of them).
+    // By chance, two launches that come at the same moment each hold a part of
+    // the chip; where something holds it for good, the wait's 5 ms are spread
+    // over ever more solves.  Contexts on threads of their own, ms per step
+    // of any of them, by launches -> in one launch: two of 223 work-groups
+    // 1.15 -> 0.22; three 0.90 -> 0.28 (5 of 900 solves handed over, the slowest
+    // step 6.8 -> 15.8); a batch and one of 223 3.1 -> 0.75; two FP32 ones of 193
+    // 2.5 -> 0.65; two GMRES of 193 17.3 -> 5.9.
     void hand_over()
     {
-        k.group.cooldown = 8;
+        k.group.cooldown = k.group.penalty;
+        k.group.penalty = std::min(2 * k.group.penalty, 32);
         k.group.gave_up++;
     }
+    void got_through() { k.group.penalty = 1; }
 
     // The assembled MHFEM rows are scaled so that every diagonal entry is
     // exactly 1 (LinearSystem.h:196-201, BoundaryConditions.hpp:200-203,
@@ -3041,6 +3051,7 @@ struct Solve {
                     group_clear_failed(c, k.sc.p, k.nseg);
                     break;
                 }
+                got_through();
                 if (all_done()) return most_iterations();
                 if (!any_restart()) break;
                 bicg_init<T>(b, x, v, M_RESTART);
@@ -3167,6 +3178,8 @@ struct Solve {
                 if (k.h_sc[S_FAIL] != 0.0) {
                     hand_over();  // on with launches, from the replaced residual
                     group_clear_failed(c, k.sc.p, 1);
+                } else {
+                    got_through();
                 }
             } else {
                 if (continued)
@@ -3322,6 +3335,7 @@ int Solve::gmres(const double *b, double *x, double tol, int maxit, int m, doubl
                 hipLaunchKernelGGL(k_set_slot, 1, 64, 0, c.stream, k.sc.p, (int)S_FAIL, 0.0);
                 MHFEM_HIP(hipGetLastError());
             } else {
+                got_through();
                 it = (int)k.h_sc[S_IT];
             }
             beta = norm;
