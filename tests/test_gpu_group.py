@@ -191,6 +191,77 @@ def test_no_round_behind_the_end_of_a_solve():
     s.close()
 
 
+@pytest.mark.parametrize("graph", [False, True])
+def test_a_batch_that_gives_up_hands_over(graph):
+    """The same in a batch, where the launched iteration then narrows to the
+    instances still running, and in captured steps, which are captured again
+    with and without iterations."""
+    members = [problems.ensemble_member(sd, 500 + k) for k, sd in enumerate([14, 30, 22, 3, 40, 26, 9])]
+    batch = problems.concatenate(members)
+    s = capi.Solver(batch, tol=1e-13)
+    co, fo = s.batch_info()
+    oracles = [pyoracle.Oracle(m) for m in members]
+    t = 0.0
+    for k, ticks in enumerate([500000, 0, 0, 0, 500000, 500000]):
+        print(f"\n[group] batch, graph {graph}, step {k}, bound {ticks}", flush=True)
+        _group.wait_bound(s, ticks)
+        before = _group.info(s)
+        (s.step_graph if graph else s.step)(t, batch.dt)
+        i = _group.info(s)
+        # in one launch; two tries that give up; by launches; in one launch
+        assert i["gave_up"] - before["gave_up"] == (k in (1, 2)), (k, i)
+        assert (i["launches"] > before["launches"]) == (k != 3), (k, i)
+        z, zk = s.get_array("Z_iF"), s.get_array("Z_iK")
+        for j, (m, o) in enumerate(zip(members, oracles)):
+            o.step(t, m.dt, tol=1e-13)
+            assert rel(z[fo[j]:fo[j + 1]], o.array("Z_iF")) < 1e-10, (k, j)
+            assert rel(zk[co[j]:co[j + 1]], o.array("Z_iK")) < 1e-10, (k, j)
+        t += batch.dt
+    s.close()
+
+
+@pytest.mark.parametrize("precision", ["fp64", "fp32-refined", "fp32-reliable"])
+@pytest.mark.parametrize("limit", [1, 2, 7])
+def test_iteration_limit_inside_the_launch(limit, precision):
+    """A solve that stops at max_iterations stops there in both forms, with
+    the same iterate up to the rounding of a few iterations (FP32: of its
+    6e-8 numbers)."""
+    pr = problems.adr_3d(s=6, n=2, preconditioner="diagonal")
+    b = np.random.default_rng(1).standard_normal(pr.n * pr.num_faces)
+    out = []
+    for off in (False, True):
+        s = capi.Solver(pr, preconditioner="diagonal", tol=1e-12, precision=precision, inner_tol=1e-4,
+                        max_iterations=limit)
+        _group.launched(s, off)
+        s.preIterate(0.0, pr.dt)
+        s.assembleLinearSystem(0.0, pr.dt)
+        out.append(s.solve_rhs(b, np.zeros_like(b)))
+        s.close()
+    (x, st), (y, su) = out
+    assert not st.converged and not su.converged
+    assert st.iterations == su.iterations == limit
+    assert np.linalg.norm(x - y) <= (1e-10 if precision == "fp64" else 1e-4) * np.linalg.norm(y)
+
+
+def test_breakdown_inside_the_launch():
+    """Values on Dirichlet faces only, from zero, in FP64: (r, r*) is zero
+    after the first iteration, the launch ends, the host restarts it."""
+    pr = problems.adr_2d(s=18)
+    x = []
+    for off in (False, True):
+        s = capi.Solver(pr, preconditioner="diagonal", tol=1e-13)
+        _group.launched(s, off)
+        s.preIterate(0.0, pr.dt)
+        s.assembleLinearSystem(0.0, pr.dt)
+        _, _, _, rhs = s.export_system()
+        z, st = s.solve_rhs(rhs, np.zeros_like(rhs))
+        i = _group.info(s)
+        assert st.converged and i["gave_up"] == 0 and (i["launches"] == 0 if off else i["launches"] >= 2), i
+        x.append(z)
+        s.close()
+    assert rel(x[0], x[1]) < 1e-10
+
+
 def test_batch_larger_than_the_chip():
     """More work-groups than fit at once: segments start in turn."""
     members = [problems.ensemble_member(sd, 40 + k) for k, sd in enumerate([150, 20, 90, 150, 150, 7, 150])]
