@@ -52,14 +52,18 @@ namespace mhfem {
 
 constexpr int GROUP_ROT = 4;  // rotating copies of the published vectors and partial sums
 constexpr int GROUP_REP = 8;  // copies of the partial sums, each read by every 8th work-group
-// Pause before the first look at the others' values, in 64 cycles (0.48 us at
+// Pause before the first look at the others' values, in 64 cycles (0.53 us at
 // 2.4 GHz).  They cannot be there sooner than a store and a load take, and
-// looks before that only load the fabric that carries them: us per iteration
-// with 0 / 12 / 16 / 20 / 24 / 40: 114,000 faces 7.1 / 5.7 / 4.9 / 5.1 / 5.3 /
-// 6.1; the 32 ragged instances 18.0 / 14.9 / 13.9 / 12.5 / 12.8 / 14.6 ms; 12,400
-// faces 6.4 / 6.2 / 6.1 / 6.3 / 6.5 / 7.4.  Later looks gain nothing from longer
-// pauses (4 or 8 instead of 1: 2-20 % slower).
-constexpr int GROUP_FIRST_LOOK = 18;
+// looks before that only load the fabric that carries them: ms per pass with
+// 0 / 12 / 16 / 18 / 19 / 20 / 21 / 22 / 24 (the shorter the code between post
+// and look, the longer the best pause): 114,000 faces of tetrahedra, 359
+// iterations 2.83 / 2.32 / 2.02 / 1.90 / 1.89 / 1.89 / 1.92 / 1.94 / 1.98; 121,600
+// of triangles, 132 iterations 1.36 / 1.12 / 1.02 / 0.96 / 0.91 / 0.86 / 0.85 /
+// 0.84 / 0.86; FP32, 98,400 faces n = 2, 958 iterations 10.0 / 8.84 / 8.19 / 7.85 /
+// 7.77 / 7.74 / 7.82 / 7.80 / 7.99; 32 ragged instances 18.1 / 15.6 / 14.2 / 14.1 /
+// 14.2 / 14.3 / 14.5 / 14.6 / 14.9.  Later looks gain nothing from longer pauses
+// (4 or 8 instead of 1: 2-20 % slower).
+constexpr int GROUP_FIRST_LOOK = 20;
 constexpr int GROUP_ND = 4;   // dot products of a reduction, at most
 
 // partial sums a wavefront adds, per dot product: BS / 256 wavefronts for each
@@ -301,11 +305,12 @@ __device__ __forceinline__ bool bicg_share(const SellView<T> &A, const GroupView
     }
     double rho = uniform(sc[S_RHO]), rho_old = uniform(sc[S_RHO_OLD]), alpha = uniform(sc[S_ALPHA]),
            omega = uniform(sc[S_OMEGA]), beta = uniform(sc[S_BETA]);
-    double resid = 0.0, it = uniform(sc[S_IT]), brk = uniform(sc[S_BREAK]);
+    double resid = 0.0;
+    int it = __builtin_amdgcn_readfirstlane((int)sc[S_IT]);
+    bool brk = uniform(sc[S_BREAK]) != 0.0, done = false, restart = false;
     double inv_pap = 0.0;  // alpha / rho
-    const double bnorm = uniform(sc[S_BNORM]), tol = uniform(sc[S_TOL]), maxit = uniform(sc[S_MAXIT]),
-                 rast_sq = uniform(sc[S_RAST_SQ]);
-    double done = 0.0, restart = 0.0;
+    const double bnorm = uniform(sc[S_BNORM]), tol = uniform(sc[S_TOL]), rast_sq = uniform(sc[S_RAST_SQ]);
+    const int maxit = __builtin_amdgcn_readfirstlane((int)sc[S_MAXIT]);
     const double eps2 = 2.220446049250313e-16 * 2.220446049250313e-16;
     // every read of the arrays that the segment's work-groups write at the
     // end is complete before this work-group's first partial sums go out
@@ -355,19 +360,16 @@ __device__ __forceinline__ bool bicg_share(const SellView<T> &A, const GroupView
         if ((lane & (64 / ND - 1)) == 0) part[par][lane / (64 / ND)][wid] = ws;
         __syncthreads();
         if (tid < parts * ND * GROUP_REP) {
-            const int h = NP > 1 ? tid / (ND * GROUP_REP) : 0;
-            const double *w = part[par][tid % ND] + h * (PT / 64);
-            double s = w[0];
+            const int h = NP > 1 ? tid / (ND * GROUP_REP) : 0, rep = NP > 1 ? tid / ND % GROUP_REP : tid / ND;
+            double s = part[par][tid % ND][h * (PT / 64)];
 #pragma unroll
-            for (int q = 1; q < PT / 64; q++) s += w[q];
+            for (int q = 1; q < PT / 64; q++) s += part[par][tid % ND][h * (PT / 64) + q];
             if (is_sentinel(s)) s = __builtin_nan("");
-            coherent_store(slots + (((int64_t)(tid / ND % GROUP_REP) * GROUP_ROT + rot) * GROUP_ND + tid % ND) * G +
-                               task.rank + h,
-                           s);
+            coherent_store(slots + (((int64_t)rep * GROUP_ROT + rot) * GROUP_ND + tid % ND) * G + task.rank + h, s);
         }
 #pragma unroll
         for (int k = 0; k < W; k++)
-            if (col[k] < 0) nb[k] = mine[par][-1 - col[k]];
+            nb[k] = mine[par][min((unsigned)~col[k], (unsigned)BS)];  // (zeros until a remote one is there)
         // Polls for the neighbours' values in other work-groups and, in wave
         // d + ND c, for the sums of dot d of SLOTS work-groups: each round looks
         // at everything still missing with one wait.
@@ -421,11 +423,12 @@ __device__ __forceinline__ bool bicg_share(const SellView<T> &A, const GroupView
         // previous one: its copies are cleared, for epoch e + 3
         const int old = (e + GROUP_ROT - 1) & (GROUP_ROT - 1);
         if (shared_face) unpublish<T, N>(pub + (int64_t)old * g.rows + (int64_t)at * N);
-        if (tid < parts * GROUP_ND * GROUP_REP)
-            coherent_store(slots +
-                               (((int64_t)(tid / GROUP_ND % GROUP_REP) * GROUP_ROT + old) * GROUP_ND + tid % GROUP_ND) * G +
-                               task.rank + (NP > 1 ? tid / (GROUP_ND * GROUP_REP) : 0),
+        if (tid < parts * GROUP_ND * GROUP_REP) {
+            const int h = NP > 1 ? tid / (GROUP_ND * GROUP_REP) : 0,
+                      rep = NP > 1 ? tid / GROUP_ND % GROUP_REP : tid / GROUP_ND;
+            coherent_store(slots + (((int64_t)rep * GROUP_ROT + old) * GROUP_ND + tid % GROUP_ND) * G + task.rank + h,
                            sentinel_value<double>());
+        }
         e++;
         return s_fail == 0;
     };
@@ -457,19 +460,19 @@ __device__ __forceinline__ bool bicg_share(const SellView<T> &A, const GroupView
             const double D0 = total(0), D1 = total(1);
             resid = uniform(sqrt(D1) / bnorm);
             if (!(resid >= tol) || it >= maxit) {
-                done = 1.0;
+                done = true;
                 break;
             }
-            if (brk != 0.0) {
-                brk = 0.0;
-                restart = 1.0;
+            if (brk) {
+                brk = false;
+                restart = true;
                 break;
             }
             const double a = uniform(rho / D0);
             if (!(fabs(D0) > 0.0) || !isfinite(a)) {
-                restart = 1.0;
-                it += 1.0;
-                if (it >= maxit) done = 1.0;
+                restart = true;
+                it++;
+                if (it >= maxit) done = true;
                 break;
             }
             alpha = a;
@@ -504,12 +507,12 @@ __device__ __forceinline__ bool bicg_share(const SellView<T> &A, const GroupView
             const double om = uniform(D[1] > 0 ? D[0] / D[1] : 0.0), inv_om = uniform(D[1] / D[0]);
             const double rn_ = uniform(fmadd(-om, D[2], D[3]));
             omega = om;
-            it += 1.0;
+            it++;
             rho_old = rho;
             rho = rn_;
             if (!(fabs(rho) >= eps2 * rast_sq) || om == 0.0) {
                 beta = 0.0;
-                brk = 1.0;
+                brk = true;
             } else {
                 beta = uniform((rho * inv_pap) * inv_om);
             }
