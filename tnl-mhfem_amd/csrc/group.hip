@@ -33,15 +33,16 @@
 //   from the iterate it has (and keeps to that for some solves where the
 //   next try gives up too).
 //
-// Measured (MI355X, whole trajectories as in perf/cases.py, launched -> one
-// launch): 64 x 64 x 2 triangles, 3 steps 3.21 -> 0.55 ms; 201 x 201 x 2,
-// 2 steps 6.37 -> 1.05 ms; 21^3 x 6 tetrahedra n = 1, 2 steps 17.7 -> 1.94 ms
-// (48 -> 4.9 us per iteration); 20^3 x 6 n = 2, FP32, 6 steps 50.5 -> 10.3 ms;
-// 20^3 voxels n = 3, 6.77 -> 1.33 ms; 32 ragged 2-D instances 40.8 -> 13.2 ms.  An exchange takes 2.4 us with 200
-// work-groups: 0.5 us of arithmetic, 0.4 us of work-group sums, the rest from
-// the post of the slowest work-group to its sum in every other one.  Tried:
-// neighbours polled only after the sums are in (10 us per iteration where 8
-// were needed then); faces in the mesh order (gathers 2.3 us instead of 1.6).
+// Measured (MI355X, whole trajectories as in perf/cases.py, ms, and us per
+// iteration, by launches -> in one launch): 64 x 64 x 2 triangles, 3 steps 1.82 ->
+// 0.48 (31 -> 8.1); 201 x 201 x 2, 2 steps 3.94 -> 0.86 (26 -> 6.5); 21^3 x 6
+// tetrahedra n = 1, 2 steps 9.8 -> 1.89 (27 -> 5.3); 20^3 x 6 n = 2, FP32, 6 steps
+// 32.9 -> 7.7 (34 -> 8.0); 20^3 voxels n = 3, 3.53 -> 1.23 (32 -> 11); 32 ragged 2-D
+// instances 36.4 -> 14.4.  An exchange takes 2.4 us with 200 work-groups: 0.5 us
+// of arithmetic, 0.4 us of work-group sums, the rest from the post of the
+// slowest work-group to its sum in every other one.  Tried: neighbours polled
+// only after the sums are in (10 us per iteration where 8 were needed then);
+// faces in the mesh order (gathers 2.3 us instead of 1.6).
 #include <algorithm>
 #include <type_traits>
 
@@ -521,7 +522,8 @@ __device__ __forceinline__ bool bicg_share(const SellView<T> &A, const GroupView
         Pack<T, N> x = own[0][tid];
 #pragma unroll
         for (int i = 0; i < N; i++) {
-            x.v[i] += fmadd(al, p.v[i], om * s.v[i]);
+            // (n = 1 rounds the other product first: the bits these solves have had)
+            x.v[i] += N == 1 ? fmadd(om, s.v[i], al * p.v[i]) : fmadd(al, p.v[i], om * s.v[i]);
             r.v[i] = fmadd(-om, As.v[i], s.v[i]);
             p.v[i] = fmadd(be, fmadd(-om, Ap.v[i], p.v[i]), r.v[i]);
         }
@@ -583,9 +585,9 @@ __global__ void __launch_bounds__(BS) k_bicg_group(SellView<T> A, GroupView g, T
 // Givens rotations are done by one lane of every work-group, the same numbers
 // in each.  The launched form takes ten launches and three host reads per
 // iteration.  Measured at 197,000 unknowns (20^3 x 6 tetrahedra, n = 2,
-// m = 30): 118 -> 24 us per iteration, the step 49.9 -> 9.7 ms; about 8 us of
-// an iteration are the three exchanges, the rest the four passes over V and
-// the rotations.
+// m = 30): 115 -> 24 us per iteration, the step 37.5 -> 7.8 ms (326
+// iterations); about 8 us of an iteration are the three exchanges, the rest the
+// four passes over V and the rotations.
 constexpr int GMRES_M = 32;
 
 struct GmresArgs {
