@@ -306,12 +306,11 @@ __device__ __forceinline__ bool bicg_share(const SellView<T> &A, const GroupView
     }
     double rho = uniform(sc[S_RHO]), rho_old = uniform(sc[S_RHO_OLD]), alpha = uniform(sc[S_ALPHA]),
            omega = uniform(sc[S_OMEGA]), beta = uniform(sc[S_BETA]);
-    double resid = 0.0;
-    int it = __builtin_amdgcn_readfirstlane((int)sc[S_IT]);
-    bool brk = uniform(sc[S_BREAK]) != 0.0, done = false, restart = false;
+    double resid = 0.0, it = uniform(sc[S_IT]), brk = uniform(sc[S_BREAK]);
     double inv_pap = 0.0;  // alpha / rho
-    const double bnorm = uniform(sc[S_BNORM]), tol = uniform(sc[S_TOL]), rast_sq = uniform(sc[S_RAST_SQ]);
-    const int maxit = __builtin_amdgcn_readfirstlane((int)sc[S_MAXIT]);
+    const double bnorm = uniform(sc[S_BNORM]), tol = uniform(sc[S_TOL]), maxit = uniform(sc[S_MAXIT]),
+                 rast_sq = uniform(sc[S_RAST_SQ]);
+    double done = 0.0, restart = 0.0;
     const double eps2 = 2.220446049250313e-16 * 2.220446049250313e-16;
     // every read of the arrays that the segment's work-groups write at the
     // end is complete before this work-group's first partial sums go out
@@ -360,8 +359,19 @@ __device__ __forceinline__ bool bicg_share(const SellView<T> &A, const GroupView
         const double ws = sums_wave<ND>(acc);
         if ((lane & (64 / ND - 1)) == 0) part[par][lane / (64 / ND)][wid] = ws;
         __syncthreads();
-        if (tid < parts * ND * GROUP_REP) {
-            const int h = NP > 1 ? tid / (ND * GROUP_REP) : 0, rep = NP > 1 ? tid / ND % GROUP_REP : tid / ND;
+        // (The two forms are apart for the compiler's sake: with the second for
+        // both, the kernels of one part are 1-2 % slower.)
+        if constexpr (NP == 1) {
+            if (tid < ND * GROUP_REP) {
+                double s = part[par][tid % ND][0];
+#pragma unroll
+                for (int q = 1; q < NW; q++) s += part[par][tid % ND][q];
+                if (is_sentinel(s)) s = __builtin_nan("");
+                coherent_store(slots + (((int64_t)(tid / ND) * GROUP_ROT + rot) * GROUP_ND + tid % ND) * G + task.rank,
+                               s);
+            }
+        } else if (tid < parts * ND * GROUP_REP) {
+            const int h = tid / (ND * GROUP_REP), rep = tid / ND % GROUP_REP;
             double s = part[par][tid % ND][h * (PT / 64)];
 #pragma unroll
             for (int q = 1; q < PT / 64; q++) s += part[par][tid % ND][h * (PT / 64) + q];
@@ -461,19 +471,19 @@ __device__ __forceinline__ bool bicg_share(const SellView<T> &A, const GroupView
             const double D0 = total(0), D1 = total(1);
             resid = uniform(sqrt(D1) / bnorm);
             if (!(resid >= tol) || it >= maxit) {
-                done = true;
+                done = 1.0;
                 break;
             }
-            if (brk) {
-                brk = false;
-                restart = true;
+            if (brk != 0.0) {
+                brk = 0.0;
+                restart = 1.0;
                 break;
             }
             const double a = uniform(rho / D0);
             if (!(fabs(D0) > 0.0) || !isfinite(a)) {
-                restart = true;
-                it++;
-                if (it >= maxit) done = true;
+                restart = 1.0;
+                it += 1.0;
+                if (it >= maxit) done = 1.0;
                 break;
             }
             alpha = a;
@@ -508,12 +518,12 @@ __device__ __forceinline__ bool bicg_share(const SellView<T> &A, const GroupView
             const double om = uniform(D[1] > 0 ? D[0] / D[1] : 0.0), inv_om = uniform(D[1] / D[0]);
             const double rn_ = uniform(fmadd(-om, D[2], D[3]));
             omega = om;
-            it++;
+            it += 1.0;
             rho_old = rho;
             rho = rn_;
             if (!(fabs(rho) >= eps2 * rast_sq) || om == 0.0) {
                 beta = 0.0;
-                brk = true;
+                brk = 1.0;
             } else {
                 beta = uniform((rho * inv_pap) * inv_om);
             }
@@ -901,8 +911,8 @@ __global__ void __launch_bounds__(BS) k_gmres_group(SellView<double> A, GroupVie
     }
 }
 
-// sentinels in the published vectors and the slots, counters at zero; a
-// single segment that has stopped (sc) needs the counters only
+// sentinels in the published vectors and the slots, counters at zero; where
+// the segment (sc) has stopped already, the counters only
 template <typename T>
 __global__ void __launch_bounds__(256) k_group_prepare(int64_t pubn, T *pub, int slotn, double *slots, int *ticket,
                                                        unsigned *beat, const double *sc)
@@ -1173,7 +1183,7 @@ void group_iterate(Ctx &c, GroupPlan &gp, const SellView<T> &A, bool permuted, d
     unsigned *beat = reinterpret_cast<unsigned *>(gp.counters.p + 1);
     const unsigned g = (unsigned)std::min<int64_t>(1024, (std::max<int64_t>(pubn, gp.nslots) + 255) / 256);
     hipLaunchKernelGGL(k_group_prepare<T>, g, 256, 0, c.stream, pubn, pub, gp.nslots, gp.slots.p, ticket, beat,
-                       gp.batch ? (const double *)nullptr : (const double *)sc);
+                       q ? (const double *)sc : (const double *)nullptr);
     const GroupView v{gp.total, c.rows, gp.task.p, face, pos, reinterpret_cast<const int2 *>(gp.seg.p),
                       ticket, beat, gp.slots.p, sc, gp.wait_ticks};
     with_bicg_group<T>(gp.threads, c.n, gp.width, gp.lds, gp.batch, [&](auto *kernel, int threads) {
