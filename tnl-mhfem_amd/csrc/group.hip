@@ -35,10 +35,10 @@
 //
 // Measured (MI355X, whole trajectories as in perf/cases.py, ms, and us per
 // iteration, by launches -> in one launch): 64 x 64 x 2 triangles, 3 steps 1.82 ->
-// 0.48 (31 -> 8.1); 201 x 201 x 2, 2 steps 3.94 -> 0.86 (26 -> 6.5); 21^3 x 6
-// tetrahedra n = 1, 2 steps 9.8 -> 1.89 (27 -> 5.3); 20^3 x 6 n = 2, FP32, 6 steps
-// 32.9 -> 7.7 (34 -> 8.0); 20^3 voxels n = 3, 3.53 -> 1.23 (32 -> 11); 32 ragged 2-D
-// instances 36.4 -> 14.4.  An exchange takes 2.4 us with 200 work-groups: 0.5 us
+// 0.48 (31 -> 8.1); 201 x 201 x 2, 2 steps 3.94 -> 0.84 (26 -> 6.4); 21^3 x 6
+// tetrahedra n = 1, 2 steps 9.8 -> 1.87 (27 -> 5.2); 20^3 x 6 n = 2, FP32, 6 steps
+// 32.9 -> 7.7 (34 -> 8.0); 20^3 voxels n = 3, 3.53 -> 1.20 (32 -> 11); 32 ragged 2-D
+// instances 36.4 -> 14.2.  An exchange takes 2.4 us with 200 work-groups: 0.5 us
 // of arithmetic, 0.4 us of work-group sums, the rest from the post of the
 // slowest work-group to its sum in every other one.  Tried: neighbours polled
 // only after the sums are in (10 us per iteration where 8 were needed then);
@@ -56,13 +56,12 @@ constexpr int GROUP_REP = 8;  // copies of the partial sums, each read by every 
 // Pause before the first look at the others' values, in 64 cycles (0.53 us at
 // 2.4 GHz).  They cannot be there sooner than a store and a load take, and
 // looks before that only load the fabric that carries them: ms per pass with
-// 0 / 12 / 16 / 18 / 19 / 20 / 21 / 22 / 24 (the shorter the code between post
-// and look, the longer the best pause): 114,000 faces of tetrahedra, 359
-// iterations 2.83 / 2.32 / 2.02 / 1.90 / 1.89 / 1.89 / 1.92 / 1.94 / 1.98; 121,600
-// of triangles, 132 iterations 1.36 / 1.12 / 1.02 / 0.96 / 0.91 / 0.86 / 0.85 /
-// 0.84 / 0.86; FP32, 98,400 faces n = 2, 958 iterations 10.0 / 8.84 / 8.19 / 7.85 /
-// 7.77 / 7.74 / 7.82 / 7.80 / 7.99; 32 ragged instances 18.1 / 15.6 / 14.2 / 14.1 /
-// 14.2 / 14.3 / 14.5 / 14.6 / 14.9.  Later looks gain nothing from longer pauses
+// 0 / 12 / 16 / 18 / 19 / 20 / 21 / 22 / 24: 114,000 faces of tetrahedra, 357
+// iterations 2.79 / 2.28 / 1.92 / 1.87 / 1.85 / 1.87 / 1.90 / 1.92 / 1.95; 121,600
+// of triangles, 131 iterations 1.35 / 1.11 / 1.01 / 0.95 / 0.87 / 0.85 / 0.84 /
+// 0.83 / 0.83; FP32, 98,400 faces n = 2, 958 iterations 10.0 / 8.66 / 7.92 / 7.68 /
+// 7.58 / 7.67 / 7.74 / 7.77 / 7.82; 32 ragged instances 18.6 / 15.7 / 14.4 / 14.0 /
+// 14.1 / 14.3 / 14.4 / 14.6 / 14.8.  Later looks gain nothing from longer pauses
 // (4 or 8 instead of 1: 2-20 % slower).
 constexpr int GROUP_FIRST_LOOK = 20;
 constexpr int GROUP_ND = 4;   // dot products of a reduction, at most
